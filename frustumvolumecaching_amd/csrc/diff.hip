@@ -65,7 +65,9 @@ enum {
   B_W3T = 192,  // 4 x 4
   B_W2T = 208,  // 4 x 16
   B_W1T = 272,  // 2 blocks (encoding, quad-level order) x 16
-  N_DIFF_FRAGS = 304
+  N_DIFF_FRAGS = 304,
+  N_FWD_FRAGS = 160,             // the forward's fragments come first
+  N_HEAD_FRAGS = B_W3T - F_H1    // the colour MLP's, forward and backward
 };
 
 // k index of slot m in lane group g
@@ -83,7 +85,9 @@ static int row_enc(int nb, int i) { return k_enc(4 * nb + (i % 4), i / 4); }
 static int row_head(int i) { return k_head(i % 4, i / 4); }
 
 // Index of every fragment value in the concatenated parameters
-// [mlp_base | mlp_head] (-1: zero).
+// [mlp_base | mlp_head] (-1: zero).  Fragments f .. f + 3 (f a multiple of 4,
+// slots m .. m + 3 of one block) lie together per lane, so a lane reads four
+// slots' operands with one 16-byte load.
 std::vector<int> diff_frag_index() {
   const int n_base = 32 * 64 + 64 * 64 + 64 * 16;
   const int W1 = 0, W2 = 32 * 64, W3 = 32 * 64 + 64 * 64, H1 = n_base, H2 = n_base + 32 * 64;
@@ -91,7 +95,10 @@ std::vector<int> diff_frag_index() {
   auto put = [&](int f0, int n_blocks, int n_slots, auto val) {
     for (int nb = 0; nb < n_blocks; nb++)
       for (int m = 0; m < n_slots; m++)
-        for (int lane = 0; lane < 64; lane++) t[((size_t)(f0 + nb * n_slots + m)) * 64 + lane] = val(nb, m, lane % 16, lane / 16);
+        for (int lane = 0; lane < 64; lane++) {
+          const size_t f = (size_t)(f0 + nb * n_slots + m);
+          t[((f >> 2) * 64 + lane) * 4 + (f & 3)] = val(nb, m, lane % 16, lane / 16);
+        }
   };
   // forward: A = W[16 nb + i][k(m, g)]
   put(F_W1, 4, 8, [&](int nb, int m, int i, int g) { return W1 + (16 * nb + i) * 32 + k_enc(m, g); });
@@ -120,19 +127,31 @@ __global__ void k_diff_pack(const int* __restrict__ idx, const float* __restrict
 __device__ __forceinline__ f4 mma4(float a, float b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-// NB output blocks from M input slots with fragments fr[(nb * M + m) * 64]
-// (the lane index is made opaque per call so the fragment loads of one layer
-// are issued together but not hoisted across layers)
+// NB output blocks from M input slots with the fragments of a layer at fr (in
+// LDS; slots 4q..4q+3 of block nb at fr[(nb * M / 4 + q) * 64 + lane]).  The
+// lane index is made opaque per call so that the reads of a layer are not
+// hoisted into registers across the sample loop.
 template <int NB, int M>
-__device__ __forceinline__ void dense4(const float* __restrict__ fr, int lane_, const float* x, f4* y) {
+__device__ __forceinline__ void dense4(const float4* fr, int lane_, const float* x, f4* y) {
   const int lane = opaque(lane_);
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) {
     f4 acc = f4zero();
 #pragma unroll
-    for (int m = 0; m < M; m++) acc = mma4(fr[(nb * M + m) * 64 + lane], x[m], acc);
+    for (int q = 0; q < M / 4; q++) {
+      const float4 a = fr[(nb * (M / 4) + q) * 64 + lane];
+      acc = mma4(a.x, x[4 * q], acc);
+      acc = mma4(a.y, x[4 * q + 1], acc);
+      acc = mma4(a.z, x[4 * q + 2], acc);
+      acc = mma4(a.w, x[4 * q + 3], acc);
+    }
     y[nb] = acc;
   }
+}
+// the fragments [f0, f0 + n) of the packed table into LDS (every thread of the block)
+__device__ __forceinline__ void stage_diff_frags(const float* __restrict__ frags, int f0, int n, float4* lds) {
+  const float4* src = reinterpret_cast<const float4*>(frags) + f0 * 16;
+  for (int i = threadIdx.x; i < n * 16; i += blockDim.x) lds[i] = src[i];
 }
 template <int NB> __device__ __forceinline__ void relu_slots(const f4* y, float* x) {
 #pragma unroll
@@ -219,8 +238,9 @@ struct FwdActs {
 
 // colour MLP on the base-output rows 4g..4g+3 in `rows` (rows 1..8 are the
 // latents; row 0 and rows 9..15 give way to the 1.0 padding inputs)
-__device__ __forceinline__ void head_forward(const float* __restrict__ fr, int lane, int g, f4 rows, V3 d01,
-                                             FwdActs& a) {
+// fr: the staged fragments from fragment F0 on
+template <int F0>
+__device__ __forceinline__ void head_forward(const float4* fr, int lane, int g, f4 rows, V3 d01, FwdActs& a) {
   float sh[4], h[16];
   sh4_quarter_f32(d01, g, sh);
 #pragma unroll
@@ -229,12 +249,12 @@ __device__ __forceinline__ void head_forward(const float* __restrict__ fr, int l
     a.xh[m] = (r >= 1 && r <= 8) ? rows[m] : 1.0f;
     a.xh[4 + m] = sh[m];
   }
-  dense4<4, 8>(fr + F_H1 * 64, lane, a.xh, a.z1);
+  dense4<4, 8>(fr + (F_H1 - F0) * 16, lane, a.xh, a.z1);
   relu_slots<4>(a.z1, h);
-  dense4<1, 16>(fr + F_H2 * 64, lane, h, &a.o);
+  dense4<1, 16>(fr + (F_H2 - F0) * 16, lane, h, &a.o);
 }
 
-__device__ __forceinline__ void net_forward(const float* __restrict__ fr, const float* __restrict__ table,
+__device__ __forceinline__ void net_forward(const float4* fr, const float* __restrict__ table,
                                             const GridLevel* __restrict__ lv, const GridParams& gp, V3 p, V3 d01,
                                             int lane, int g, FwdActs& a) {
   uint32_t idx[4][8];
@@ -254,12 +274,12 @@ __device__ __forceinline__ void net_forward(const float* __restrict__ fr, const 
     a.enc[2 * j + 1] = e1;
   }
   float h[16];
-  dense4<4, 8>(fr + F_W1 * 64, lane, a.enc, a.a1);
+  dense4<4, 8>(fr + F_W1 * 16, lane, a.enc, a.a1);
   relu_slots<4>(a.a1, h);
-  dense4<4, 16>(fr + F_W2 * 64, lane, h, a.a2);
+  dense4<4, 16>(fr + F_W2 * 16, lane, h, a.a2);
   relu_slots<4>(a.a2, h);
-  dense4<1, 16>(fr + F_W3 * 64, lane, h, &a.out);
-  head_forward(fr, lane, g, a.out, d01, a);
+  dense4<1, 16>(fr + F_W3 * 16, lane, h, &a.out);
+  head_forward<0>(fr, lane, g, a.out, d01, a);
 }
 
 __device__ __forceinline__ V3 ray_dir01(const RayState& r) { return unit_to_01(V3{r.dx, r.dy, r.dz}); }
@@ -329,7 +349,9 @@ __global__ __launch_bounds__(256) void k_diff_net_fwd(int n, const int* __restri
                                                       const float* __restrict__ table, GridParams gp,
                                                       const float* __restrict__ frags, float4* __restrict__ out4) {
   __shared__ GridLevel lv[MAX_LEVELS];
+  __shared__ float4 fr[N_FWD_FRAGS * 16];
   if (threadIdx.x < MAX_LEVELS) lv[threadIdx.x] = gp.lv[threadIdx.x];
+  stage_diff_frags(frags, 0, N_FWD_FRAGS, fr);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
@@ -341,7 +363,7 @@ __global__ __launch_bounds__(256) void k_diff_net_fwd(int n, const int* __restri
     const V3 p = {s_pos[3 * sl], s_pos[3 * sl + 1], s_pos[3 * sl + 2]};
     const V3 d01 = ray_dir01(rays[s_ray[sl]]);
     FwdActs a;
-    net_forward(frags, table, lv, gp, p, d01, lane, g, a);
+    net_forward(fr, table, lv, gp, p, d01, lane, g, a);
     if (g == 0 && valid) out4[sl] = make_float4(a.o[0], a.o[1], a.o[2], a.out[0]);
   }
 }
@@ -421,45 +443,56 @@ __global__ __launch_bounds__(256) void k_diff_composite_bwd(int n, float alpha_t
 }
 
 // ------------------------------------------------------------ backward
-// gradient accumulators of one block in LDS (row-major [out][in])
-enum {
-  G_W1 = 0, G_W2 = 64 * 32, G_W3 = 64 * 32 + 64 * 64, G_H1 = 64 * 32 + 64 * 64 + 16 * 64,
-  G_H2 = G_H1 + 64 * 32, G_WORDS = G_H2 + 16 * 64
-};
-static const int STG = 20;  // LDS row stride of the transposed staging (floats)
+// where a layer's gradient starts in its parameter block (row-major [out][in])
+enum { G_W1 = 0, G_W2 = 64 * 32, G_W3 = 64 * 32 + 64 * 64, G_H1 = 0, G_H2 = 64 * 32 };
 
+// Weight gradients dW[out][in] = sum over samples of dY[out] X[in], by the
+// eight waves of a block over the block's 128 samples: every wave writes its
+// tile's dY and X to LDS as rows of samples, then the 16x16 blocks of dW are
+// shared out among the waves, each kept in a wave's registers over the whole
+// sample loop (40 blocks: 24 registers a lane) and added to the caller's
+// gradient once, at the end.  A lane reads its operands of four MFMA steps
+// (samples 16 q + 4 g .. + 3) as one float4; the row stride of 132 floats
+// spreads the 16 rows of such a read, and the four lane groups of a write,
+// over all LDS banks.
+// Bound by the f32 MFMA issue (464 steps of 32 cycles per tile with the
+// forward's recomputation); measured at 2^18 rays (14 M samples) against one
+// LDS atomic per tile and weight: training step 88.0 -> 80.3 ms, 4096 rays
+// 5.30 -> 5.05 ms.
+static const int BWD_WAVES = 8, BWD_SAMPLES = 16 * BWD_WAVES;
+static const int STG = BWD_SAMPLES + 4;  // LDS row stride (floats)
 
-// dW[n_out][n_in] += sum over the tile's 16 samples of dY[row][s] X[col][s]:
-// dY as NBY D blocks (rows 16 nb + 4 g + e), X as MX slots with column
-// kcol(m, g).  Samples are stored in LDS in the order 4 (s % 4) + s / 4 so
-// a lane reads its 4 k-steps (samples g, g+4, g+8, g+12) as one float4.
-template <int NBY, int MX, class KCol>
-__device__ __forceinline__ void wgrad(float* ys, float* xs, const f4* dY, const float* x, KCol kcol, int col, int g,
-                                      float* acc, int n_in) {
-  const int ps = 4 * (col % 4) + col / 4;
+template <int NB> __device__ __forceinline__ void stage_rows(float* rows, const f4* y, int g, int smp) {
 #pragma unroll
-  for (int nb = 0; nb < NBY; nb++)
+  for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-    for (int e = 0; e < 4; e++) ys[(16 * nb + 4 * g + e) * STG + ps] = dY[nb][e];
+    for (int e = 0; e < 4; e++) rows[(16 * nb + 4 * g + e) * STG + smp] = y[nb][e];
+}
+template <int MX, class KCol>
+__device__ __forceinline__ void stage_cols(float* rows, const float* x, KCol kcol, int g, int smp) {
 #pragma unroll
-  for (int m = 0; m < MX; m++) xs[kcol(m, g) * STG + ps] = x[m];
-  wave_sync();
-  const int n_kb = MX * 4 / 16;
-#pragma unroll
-  for (int jb = 0; jb < NBY; jb++) {
-    const float4 a = *reinterpret_cast<const float4*>(&ys[(16 * jb + col) * STG + 4 * g]);
-#pragma unroll
-    for (int kb = 0; kb < n_kb; kb++) {
-      const float4 b = *reinterpret_cast<const float4*>(&xs[(16 * kb + col) * STG + 4 * g]);
-      f4 d = mma4(a.x, b.x, f4zero());
-      d = mma4(a.y, b.y, d);
-      d = mma4(a.z, b.z, d);
-      d = mma4(a.w, b.w, d);
-#pragma unroll
-      for (int e = 0; e < 4; e++) atomicAdd(&acc[(16 * jb + 4 * g + e) * n_in + 16 * kb + col], d[e]);
-    }
+  for (int m = 0; m < MX; m++) rows[kcol(m, g) * STG + smp] = x[m];
+}
+// acc += block (jb, kb) of dY X^T over samples [16 q0, 16 q1)
+__device__ __forceinline__ void wgrad_block(const float* ys, const float* xs, int jb, int kb, int q0, int q1, int col,
+                                            int g, f4& acc) {
+  const float* yr = ys + (16 * jb + col) * STG + 4 * g;
+  const float* xr = xs + (16 * kb + col) * STG + 4 * g;
+#pragma unroll 4
+  for (int q = q0; q < q1; q++) {
+    const float4 a = *reinterpret_cast<const float4*>(yr + 16 * q);
+    const float4 b = *reinterpret_cast<const float4*>(xr + 16 * q);
+    acc = mma4(a.x, b.x, acc);
+    acc = mma4(a.y, b.y, acc);
+    acc = mma4(a.z, b.z, acc);
+    acc = mma4(a.w, b.w, acc);
   }
-  wave_sync();
+}
+// block (jb, kb) of dW added to the caller's gradient (rows of n_in)
+__device__ __forceinline__ void add_block(float* gw, int jb, int kb, int n_in, int col, int g, f4 acc) {
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    if (acc[e] != 0.0f) unsafeAtomicAdd(&gw[(16 * jb + 4 * g + e) * n_in + 16 * kb + col], acc[e]);
 }
 
 // column maps of the B slots (device copies of k_chain, k_enc, k_head)
@@ -509,46 +542,48 @@ __device__ __forceinline__ void scatter_run(float* __restrict__ g_pos, uint32_t 
 // colour MLP backward of a tile: d_o (output rows 4g..4g+3), d_z1
 // (hidden pre-activations) and d_xh (head inputs in the rows of the
 // base output, row r = latent r - 1 for r in 1..8)
-__device__ __forceinline__ void head_backward(const float* __restrict__ frags, int lane, int g, const FwdActs& a,
-                                              float4 dq, f4& d_o, f4* d_z1, f4& d_xh) {
+template <int F0>
+__device__ __forceinline__ void head_backward(const float4* fr, int lane, int g, const FwdActs& a, float4 dq,
+                                              f4& d_o, f4* d_z1, f4& d_xh) {
   d_o = g == 0 ? f4{dq.x, dq.y, dq.z, 0.0f} : f4zero();
   float x[16];
 #pragma unroll
   for (int e = 0; e < 4; e++) x[e] = d_o[e];
-  dense4<4, 4>(frags + B_H2T * 64, lane, x, d_z1);
+  dense4<4, 4>(fr + (B_H2T - F0) * 16, lane, x, d_z1);
   relu_grad<4>(a.z1, d_z1);
 #pragma unroll
   for (int nb = 0; nb < 4; nb++)
 #pragma unroll
     for (int e = 0; e < 4; e++) x[4 * nb + e] = d_z1[nb][e];
-  dense4<1, 16>(frags + B_H1T * 64, lane, x, &d_xh);
+  dense4<1, 16>(fr + (B_H1T - F0) * 16, lane, x, &d_xh);
 }
 
-__device__ __forceinline__ void head_wgrad(float* ys, float* xs, const FwdActs& a, const f4& d_o, const f4* d_z1,
-                                           int col, int g, float* acc) {
+// colour MLP weight gradients of the block's samples: wave w takes block
+// w % 4 of H2 over half w / 4 of the samples, and block (w / 2, w % 2) of H1.
+// Every thread of the block calls it; it ends with a barrier.
+struct HeadAcc { f4 h2, h1; };
+__device__ __forceinline__ void head_wgrad(float* stage, const FwdActs& a, const f4& d_o, const f4* d_z1, int wave,
+                                           int col, int g, HeadAcc& acc) {
+  const int smp = 16 * wave + col;
   float h[16];
   relu_slots<4>(a.z1, h);
-  wgrad<1, 16>(ys, xs, &d_o, h, KChain(), col, g, acc + G_H2, 64);
-  wgrad<4, 8>(ys, xs, d_z1, a.xh, KHead(), col, g, acc + G_H1, 32);
+  stage_rows<1>(stage, &d_o, g, smp);
+  stage_cols<16>(stage + 16 * STG, h, KChain(), g, smp);
+  __syncthreads();
+  wgrad_block(stage, stage + 16 * STG, 0, wave & 3, (wave >> 2) * 4, (wave >> 2) * 4 + 4, col, g, acc.h2);
+  __syncthreads();
+  stage_rows<4>(stage, d_z1, g, smp);
+  stage_cols<8>(stage + 64 * STG, a.xh, KHead(), g, smp);
+  __syncthreads();
+  wgrad_block(stage, stage + 64 * STG, wave >> 1, wave & 1, 0, BWD_WAVES, col, g, acc.h1);
+  __syncthreads();
+}
+__device__ __forceinline__ void flush_head(float* g_head, int wave, int col, int g, const HeadAcc& acc) {
+  add_block(g_head + G_H2, 0, wave & 3, 64, col, g, acc.h2);
+  add_block(g_head + G_H1, wave >> 1, wave & 1, 32, col, g, acc.h1);
 }
 
-// block accumulators into the caller's gradient blocks
-__device__ __forceinline__ void flush_grads(const float* acc, float* g_base, float* g_head) {
-  for (int k = threadIdx.x; k < G_WORDS; k += blockDim.x) {
-    const float v = acc[k];
-    if (v == 0.0f) continue;
-    if (k < G_H1) unsafeAtomicAdd(&g_base[k], v);
-    else unsafeAtomicAdd(&g_head[k - G_H1], v);
-  }
-}
-__device__ __forceinline__ void flush_head_grads(const float* acc, float* g_head) {
-  for (int k = G_H1 + threadIdx.x; k < G_WORDS; k += blockDim.x) {
-    const float v = acc[k];
-    if (v != 0.0f) unsafeAtomicAdd(&g_head[k - G_H1], v);
-  }
-}
-
-__global__ __launch_bounds__(256) void k_diff_net_bwd(int n, const int* __restrict__ list,
+__global__ __launch_bounds__(64 * BWD_WAVES) void k_diff_net_bwd(int n, const int* __restrict__ list,
                                                       const float* __restrict__ s_pos,
                                                       const int* __restrict__ s_ray,
                                                       const RayState* __restrict__ rays,
@@ -557,28 +592,31 @@ __global__ __launch_bounds__(256) void k_diff_net_bwd(int n, const int* __restri
                                                       const float4* __restrict__ d_out4, float* __restrict__ g_pos,
                                                       float* __restrict__ g_base, float* __restrict__ g_head) {
   __shared__ GridLevel lv[MAX_LEVELS];
-  __shared__ float acc[G_WORDS];
-  __shared__ __attribute__((aligned(16))) float stage[4][2][64 * STG];
+  __shared__ float4 fr[N_DIFF_FRAGS * 16];
+  __shared__ __attribute__((aligned(16))) float stage[128 * STG];
   if (threadIdx.x < MAX_LEVELS) lv[threadIdx.x] = gp.lv[threadIdx.x];
-  for (int k = threadIdx.x; k < G_WORDS; k += blockDim.x) acc[k] = 0.0f;
+  stage_diff_frags(frags, 0, N_DIFF_FRAGS, fr);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
-  float* ys = stage[wave][0];
-  float* xs = stage[wave][1];
-  const int n_groups = (n + 15) / 16;
-  for (int grp = blockIdx.x * 4 + wave; grp < n_groups; grp += gridDim.x * 4) {
-    const int j = grp * 16 + col;
+  const int smp = 16 * wave + col;  // the lane's sample among the block's
+  HeadAcc acc_h{f4zero(), f4zero()};
+  f4 acc_w3 = f4zero(), acc_w2[2] = {f4zero(), f4zero()}, acc_w1 = f4zero();
+  // every wave of the block takes part in every iteration (barriers); lanes
+  // past the last sample carry zero gradients
+  for (int base = blockIdx.x * BWD_SAMPLES; base < n; base += gridDim.x * BWD_SAMPLES) {
+    const int j = base + smp;
     const bool valid = j < n;
     const int sl = list ? list[valid ? j : n - 1] : (valid ? j : n - 1);
     const float4 dq = valid ? d_out4[sl] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const V3 p = {s_pos[3 * sl], s_pos[3 * sl + 1], s_pos[3 * sl + 2]};
     const V3 d01 = ray_dir01(rays[s_ray[sl]]);
     FwdActs a;
-    net_forward(frags, table, lv, gp, p, d01, lane, g, a);
+    net_forward(fr, table, lv, gp, p, d01, lane, g, a);
     // colour MLP
     f4 d_o, d_z1[4], d_xh;
-    head_backward(frags, lane, g, a, dq, d_o, d_z1, d_xh);
+    head_backward<0>(fr, lane, g, a, dq, d_o, d_z1, d_xh);
+    head_wgrad(stage, a, d_o, d_z1, wave, col, g, acc_h);
     float x[16];
     // density MLP: output rows 4g + e (0: log density, 1..8: latents)
     f4 d_out;
@@ -589,19 +627,19 @@ __global__ __launch_bounds__(256) void k_diff_net_bwd(int n, const int* __restri
     }
     f4 d_a2[4], d_a1[4], d_enc[2];
     for (int e = 0; e < 4; e++) x[e] = d_out[e];
-    dense4<4, 4>(frags + B_W3T * 64, lane, x, d_a2);
+    dense4<4, 4>(fr + B_W3T * 16, lane, x, d_a2);
     relu_grad<4>(a.a2, d_a2);
 #pragma unroll
     for (int nb = 0; nb < 4; nb++)
 #pragma unroll
       for (int e = 0; e < 4; e++) x[4 * nb + e] = d_a2[nb][e];
-    dense4<4, 16>(frags + B_W2T * 64, lane, x, d_a1);
+    dense4<4, 16>(fr + B_W2T * 16, lane, x, d_a1);
     relu_grad<4>(a.a1, d_a1);
 #pragma unroll
     for (int nb = 0; nb < 4; nb++)
 #pragma unroll
       for (int e = 0; e < 4; e++) x[4 * nb + e] = d_a1[nb][e];
-    dense4<2, 16>(frags + B_W1T * 64, lane, x, d_enc);
+    dense4<2, 16>(fr + B_W1T * 16, lane, x, d_enc);
     // hash-grid scatter: feature slot 2j + k of level 4j + g is d_enc[j / 2][2 (j % 2) + k]
     {
       uint32_t idx[4][8];
@@ -615,17 +653,33 @@ __global__ __launch_bounds__(256) void k_diff_net_bwd(int n, const int* __restri
         for (int c = 0; c < 8; c++) scatter_run(g_pos, idx[j][c], w[j][c] * d0, w[j][c] * d1, col, valid);
       }
     }
-    // weight gradients (activations as the forward's B slots)
-    head_wgrad(ys, xs, a, d_o, d_z1, col, g, acc);
+    // density MLP weight gradients (activations as the forward's B slots)
     float h[16];
     relu_slots<4>(a.a2, h);
-    wgrad<1, 16>(ys, xs, &d_out, h, KChain(), col, g, acc + G_W3, 64);
+    stage_rows<1>(stage, &d_out, g, smp);
+    stage_cols<16>(stage + 16 * STG, h, KChain(), g, smp);
+    __syncthreads();
+    wgrad_block(stage, stage + 16 * STG, 0, wave & 3, (wave >> 2) * 4, (wave >> 2) * 4 + 4, col, g, acc_w3);
+    __syncthreads();
     relu_slots<4>(a.a1, h);
-    wgrad<4, 16>(ys, xs, d_a2, h, KChain(), col, g, acc + G_W2, 64);
-    wgrad<4, 8>(ys, xs, d_a1, a.enc, KEnc(), col, g, acc + G_W1, 32);
+    stage_rows<4>(stage, d_a2, g, smp);
+    stage_cols<16>(stage + 64 * STG, h, KChain(), g, smp);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      wgrad_block(stage, stage + 64 * STG, wave >> 1, 2 * (wave & 1) + k, 0, BWD_WAVES, col, g, acc_w2[k]);
+    __syncthreads();
+    stage_rows<4>(stage, d_a1, g, smp);
+    stage_cols<8>(stage + 64 * STG, a.enc, KEnc(), g, smp);
+    __syncthreads();
+    wgrad_block(stage, stage + 64 * STG, wave >> 1, wave & 1, 0, BWD_WAVES, col, g, acc_w1);
+    __syncthreads();
   }
-  __syncthreads();
-  flush_grads(acc, g_base, g_head);
+  flush_head(g_head, wave, col, g, acc_h);
+  add_block(g_base + G_W3, 0, wave & 3, 64, col, g, acc_w3);
+#pragma unroll
+  for (int k = 0; k < 2; k++) add_block(g_base + G_W2, wave >> 1, 2 * (wave & 1) + k, 64, col, g, acc_w2[k]);
+  add_block(g_base + G_W1, wave >> 1, wave & 1, 32, col, g, acc_w1);
 }
 
 // ------------------------------------------------------------ cached mode
@@ -799,6 +853,9 @@ __global__ __launch_bounds__(256) void k_diffc_head_fwd(int n, const int* __rest
                                                         const RayState* __restrict__ rays, CacheView cv,
                                                         const float* __restrict__ frags,
                                                         float4* __restrict__ out4) {
+  __shared__ float4 fr[(B_H2T - F_H1) * 16];
+  stage_diff_frags(frags, F_H1, B_H2T - F_H1, fr);
+  __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int n_groups = (n + 15) / 16;
@@ -811,29 +868,27 @@ __global__ __launch_bounds__(256) void k_diffc_head_fwd(int n, const int* __rest
     LookupLane L;
     lookup_f32(cv, f, g, L);
     FwdActs a;
-    head_forward(frags, lane, g, lookup_rows(L, g), d01, a);
+    head_forward<F_H1>(fr, lane, g, lookup_rows(L, g), d01, a);
     if (g == 0 && valid) out4[sl] = make_float4(a.o[0], a.o[1], a.o[2], logf(fmaxf_(L.dsum, 1e-6f)));
   }
 }
 
-__global__ __launch_bounds__(256) void k_diffc_head_bwd(int n, const int* __restrict__ list,
+__global__ __launch_bounds__(64 * BWD_WAVES) void k_diffc_head_bwd(int n, const int* __restrict__ list,
                                                         const float* __restrict__ s_pos,
                                                         const int* __restrict__ s_ray,
                                                         const RayState* __restrict__ rays, CacheView cv,
                                                         const float* __restrict__ frags,
                                                         const float4* __restrict__ d_out4,
                                                         float* __restrict__ g_head, float* __restrict__ g_pool) {
-  __shared__ float acc[G_WORDS];
-  __shared__ __attribute__((aligned(16))) float stage[4][2][64 * STG];
-  for (int k = G_H1 + threadIdx.x; k < G_WORDS; k += blockDim.x) acc[k] = 0.0f;
+  __shared__ float4 fr[N_HEAD_FRAGS * 16];
+  __shared__ __attribute__((aligned(16))) float stage[96 * STG];
+  stage_diff_frags(frags, F_H1, N_HEAD_FRAGS, fr);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
-  float* ys = stage[wave][0];
-  float* xs = stage[wave][1];
-  const int n_groups = (n + 15) / 16;
-  for (int grp = blockIdx.x * 4 + wave; grp < n_groups; grp += gridDim.x * 4) {
-    const int j = grp * 16 + col;
+  HeadAcc acc_h{f4zero(), f4zero()};
+  for (int base = blockIdx.x * BWD_SAMPLES; base < n; base += gridDim.x * BWD_SAMPLES) {
+    const int j = base + 16 * wave + col;
     const bool valid = j < n;
     const int sl = list[valid ? j : n - 1];
     const float4 dq = valid ? d_out4[sl] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -842,10 +897,10 @@ __global__ __launch_bounds__(256) void k_diffc_head_bwd(int n, const int* __rest
     LookupLane L;
     lookup_f32(cv, f, g, L);
     FwdActs a;
-    head_forward(frags, lane, g, lookup_rows(L, g), d01, a);
+    head_forward<F_H1>(fr, lane, g, lookup_rows(L, g), d01, a);
     f4 d_o, d_z1[4], d_xh;
-    head_backward(frags, lane, g, a, dq, d_o, d_z1, d_xh);
-    head_wgrad(ys, xs, a, d_o, d_z1, col, g, acc);
+    head_backward<F_H1>(fr, lane, g, a, dq, d_o, d_z1, d_xh);
+    head_wgrad(stage, a, d_o, d_z1, wave, col, g, acc_h);
     // dL/dl_i of latent i (row i + 1: lane group (i + 1) / 4, element (i + 1) % 4)
     float d_lat[8];
 #pragma unroll
@@ -863,14 +918,19 @@ __global__ __launch_bounds__(256) void k_diffc_head_bwd(int n, const int* __rest
       }
     }
   }
-  __syncthreads();
-  flush_head_grads(acc, g_head);
+  flush_head(g_head, wave, col, g, acc_h);
 }
 
 // ------------------------------------------------------------ host
 static int persistent_blocks(int64_t n_groups) {
   const int64_t blocks = (n_groups + 3) / 4;
   return (int)std::max<int64_t>(1, std::min<int64_t>(blocks, 256 * 8));
+}
+
+// blocks of the backward kernels: one per CU (their fragments and staging
+// rows fill its LDS), 128 samples per block and iteration
+static int bwd_blocks(int64_t n) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>((n + BWD_SAMPLES - 1) / BWD_SAMPLES, 256));
 }
 
 // exclusive scan of counts[0..n) into offs[0..n] (offs[n] = total)
@@ -1005,14 +1065,14 @@ void diff_backward(Renderer& r, const float* d_rgb, float* g_pos, float* g_base,
                      D.ray_out.as<float4>(), d_rgb, D.d_out4.as<float4>());
   FVC_HIP(hipGetLastError());
   if (D.n_r > 0) {
-    hipLaunchKernelGGL(k_diff_net_bwd, dim3(persistent_blocks((D.n_r + 15) / 16)), dim3(256), 0, s, (int)D.n_r,
+    hipLaunchKernelGGL(k_diff_net_bwd, dim3(bwd_blocks(D.n_r)), dim3(64 * BWD_WAVES), 0, s, (int)D.n_r,
                        D.cached ? D.list_r.as<int>() : nullptr, D.s_pos.as<float>(), D.s_ray.as<int>(),
                        D.rays.as<RayState>(), D.pos, m.grid, D.frags.as<float>(), D.d_out4.as<float4>(), g_pos,
                        g_base, g_head);
     FVC_HIP(hipGetLastError());
   }
   if (D.n_c > 0) {
-    hipLaunchKernelGGL(k_diffc_head_bwd, dim3(persistent_blocks((D.n_c + 15) / 16)), dim3(256), 0, s, (int)D.n_c,
+    hipLaunchKernelGGL(k_diffc_head_bwd, dim3(2 * bwd_blocks(D.n_c)), dim3(64 * BWD_WAVES), 0, s, (int)D.n_c,
                        D.list_c.as<int>(), D.s_pos.as<float>(), D.s_ray.as<int>(), D.rays.as<RayState>(), D.cv,
                        D.frags.as<float>(), D.d_out4.as<float4>(), g_head, g_pool);
     FVC_HIP(hipGetLastError());
