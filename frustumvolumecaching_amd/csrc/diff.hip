@@ -22,11 +22,12 @@
 //   k_diff_net_bwd per 16 samples: the forward recomputed (no activation is
 //                  stored), the chain back through the colour MLP, the
 //                  density MLP (ReLU' = [pre-activation > 0]) and the
-//                  trilinear interpolation, on MFMA with transposed-weight
-//                  fragments; weight gradients dW = sum_s dY_s X_s^T as MFMA
-//                  over the samples (operands transposed through LDS) summed
-//                  per block in LDS, then added to the caller's gradient;
-//                  hash-table gradients scattered with FP32 atomics.
+//                  encoding, on MFMA with transposed-weight fragments; weight
+//                  gradients dW = sum_s dY_s X_s^T as MFMA over the samples
+//                  (operands transposed through LDS), summed in registers,
+//                  then added to the caller's gradient;
+//   k_diff_scatter the encoding's gradients through the trilinear weights
+//                  into the hash table's gradient with FP32 atomics.
 // Samples skipped by alpha_thre and samples after termination carry no
 // gradient (the branch decisions are constants of the forward pass).
 //
@@ -511,32 +512,90 @@ struct KHead {
   }
 };
 
-// Adds (v0, v1) to entry `key` of the hash-table gradient for the 16
-// samples of a lane row (lane col = sample).  Consecutive samples of a tile
-// lie along one ray, so at the coarse levels they share corners: a
-// segmented inclusive scan over runs of equal keys sums each run, and only
-// the run's last lane issues the two FP32 atomics.
-__device__ __forceinline__ void scatter_run(float* __restrict__ g_pos, uint32_t key, float v0, float v1, int col,
-                                            bool valid) {
-  const uint32_t kprev = __shfl_up(key, 1, 16);
-  const bool vprev = __shfl_up((int)valid, 1, 16) != 0;
-  int f = (col == 0 || kprev != key || !vprev || !valid) ? 1 : 0;  // run head
+// Hash-table gradient of samples [j0, n): entry (x, y, z) of level l gets
+// w d_enc for the sample's two features.  d_enc[l][j - j0] (level rows of
+// `cap` samples) is the network backward's gradient of the encoding.
+//
+// Bound by the L2's atomics: about 21 G requests/s whatever the address
+// range, where the lanes of one instruction that touch different words of
+// one 64-byte line make one request.  So (1) a lane quad takes one sample,
+// its lanes the two x corners times the two features, whose four words lie
+// together on dense levels and, hashed, for all but the x that carry past a
+// group of 8 entries; and (2) every quad walks SCATTER_SEG consecutive
+// samples (neighbours along a ray) and keeps the sums of the cell's four
+// (y, z) rows in registers until the cell changes, so a run of samples in
+// one cell costs four requests in all.  A wave works on one level (uniform
+// index arithmetic); the levels rotate over the blocks so that each XCD gets
+// coarse and fine ones.
+static const int SCATTER_SEG = 32;
+__global__ __launch_bounds__(256) void k_diff_scatter(int j0, int n, const int* __restrict__ list,
+                                                      const float* __restrict__ s_pos, GridParams gp,
+                                                      const float* __restrict__ d_enc, int64_t cap,
+                                                      float* __restrict__ g_pos) {
+  const int blk = blockIdx.x;
+  const int l = ((blk & 15) + (blk >> 4)) & 15;
+  const GridLevel L = gp.lv[l];
+  const bool dense = (gp.dense_mask >> l) & 1u;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int xc = (lane >> 1) & 1, f = lane & 1;
+  const int64_t seg = ((int64_t)(blk >> 4) * 4 + wave) * 16 + (lane >> 2);
+  const int64_t first = j0 + seg * SCATTER_SEG;
+  const int cnt = (int)(first >= n ? 0 : (n - first < SCATTER_SEG ? n - first : SCATTER_SEG));
+  const float* de = d_enc + 2 * ((int64_t)l * cap) + f;
+  float* gl = g_pos + 2 * (size_t)L.offset + f;
+  uint32_t cx = 0u, cy = 0u, cz = 0u;
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto flush = [&] {
+    const uint32_t x = cx + (uint32_t)xc;
 #pragma unroll
-  for (int d = 1; d < 16; d <<= 1) {
-    const float u0 = __shfl_up(v0, d, 16), u1 = __shfl_up(v1, d, 16);
-    const int fu = __shfl_up(f, d, 16);
-    if (col >= d) {
-      if (!f) { v0 += u0; v1 += u1; }
-      f |= fu;
+    for (int r = 0; r < 4; r++) {
+      const uint32_t y = cy + (uint32_t)(r & 1), z = cz + (uint32_t)(r >> 1);
+      uint32_t t;
+      if (dense) {
+        t = x + y * L.res + z * L.res2;
+        t = min(t, t - L.size);  // t < 2 * size
+      } else {
+        t = (x ^ (y * 2654435761u) ^ (z * 805459861u)) & (L.size - 1u);
+      }
+      if (acc[r] != 0.0f) unsafeAtomicAdd(gl + 2 * (size_t)t, acc[r]);
+    }
+  };
+  static const int U = 4;  // samples loaded together
+  for (int k0 = 0; k0 < cnt; k0 += U) {
+    V3 p[U];
+    float d[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int64_t j = first + min(k0 + u, cnt - 1);
+      const int sl = list ? list[j] : (int)j;
+      p[u] = V3{s_pos[3 * (int64_t)sl], s_pos[3 * (int64_t)sl + 1], s_pos[3 * (int64_t)sl + 2]};
+      d[u] = de[2 * (j - j0)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + u >= cnt) break;
+      const float px = fminf_(fmaxf_(p[u].x, 0.0f), 1.0f);
+      const float py = fminf_(fmaxf_(p[u].y, 0.0f), 1.0f);
+      const float pz = fminf_(fmaxf_(p[u].z, 0.0f), 1.0f);
+      const float ax = px * L.scale + 0.5f, ay = py * L.scale + 0.5f, az = pz * L.scale + 0.5f;
+      const float fx = floorf(ax), fy = floorf(ay), fz = floorf(az);
+      const uint32_t gx = (uint32_t)(int)fx, gy = (uint32_t)(int)fy, gz = (uint32_t)(int)fz;
+      if (gx != cx || gy != cy || gz != cz) {
+        flush();
+        cx = gx; cy = gy; cz = gz;
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = 0.0f;
+      }
+      const float wx = ax - fx, wy = ay - fy, wz = az - fz;
+      const float vx = xc ? wx : 1.0f - wx, uy = 1.0f - wy, uz = 1.0f - wz;
+      const float w0 = vx * uy, w1 = vx * wy;
+      acc[0] = acc[0] + (w0 * uz) * d[u];
+      acc[1] = acc[1] + (w1 * uz) * d[u];
+      acc[2] = acc[2] + (w0 * wz) * d[u];
+      acc[3] = acc[3] + (w1 * wz) * d[u];
     }
   }
-  const uint32_t knext = __shfl_down(key, 1, 16);
-  const bool vnext = __shfl_down((int)valid, 1, 16) != 0;
-  const bool tail = col == 15 || knext != key || !vnext;
-  if (valid && tail && (v0 != 0.0f || v1 != 0.0f)) {
-    unsafeAtomicAdd(&g_pos[2 * (size_t)key], v0);
-    unsafeAtomicAdd(&g_pos[2 * (size_t)key + 1], v1);
-  }
+  flush();
 }
 
 // colour MLP backward of a tile: d_o (output rows 4g..4g+3), d_z1
@@ -583,13 +642,15 @@ __device__ __forceinline__ void flush_head(float* g_head, int wave, int col, int
   add_block(g_head + G_H1, wave >> 1, wave & 1, 32, col, g, acc.h1);
 }
 
-__global__ __launch_bounds__(64 * BWD_WAVES) void k_diff_net_bwd(int n, const int* __restrict__ list,
+// samples [j0, n) of the list; d_feat: [16 levels][cap] gradients of the encoding
+__global__ __launch_bounds__(64 * BWD_WAVES) void k_diff_net_bwd(int j0, int n, const int* __restrict__ list,
                                                       const float* __restrict__ s_pos,
                                                       const int* __restrict__ s_ray,
                                                       const RayState* __restrict__ rays,
                                                       const float* __restrict__ table, GridParams gp,
                                                       const float* __restrict__ frags,
-                                                      const float4* __restrict__ d_out4, float* __restrict__ g_pos,
+                                                      const float4* __restrict__ d_out4,
+                                                      float2* __restrict__ d_feat, int64_t cap,
                                                       float* __restrict__ g_base, float* __restrict__ g_head) {
   __shared__ GridLevel lv[MAX_LEVELS];
   __shared__ float4 fr[N_DIFF_FRAGS * 16];
@@ -604,7 +665,7 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_diff_net_bwd(int n, const in
   f4 acc_w3 = f4zero(), acc_w2[2] = {f4zero(), f4zero()}, acc_w1 = f4zero();
   // every wave of the block takes part in every iteration (barriers); lanes
   // past the last sample carry zero gradients
-  for (int base = blockIdx.x * BWD_SAMPLES; base < n; base += gridDim.x * BWD_SAMPLES) {
+  for (int base = j0 + blockIdx.x * BWD_SAMPLES; base < n; base += gridDim.x * BWD_SAMPLES) {
     const int j = base + smp;
     const bool valid = j < n;
     const int sl = list ? list[valid ? j : n - 1] : (valid ? j : n - 1);
@@ -640,18 +701,11 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_diff_net_bwd(int n, const in
 #pragma unroll
       for (int e = 0; e < 4; e++) x[4 * nb + e] = d_a1[nb][e];
     dense4<2, 16>(fr + B_W1T * 16, lane, x, d_enc);
-    // hash-grid scatter: feature slot 2j + k of level 4j + g is d_enc[j / 2][2 (j % 2) + k]
-    {
-      uint32_t idx[4][8];
-      float w[4][8];
-      quad_corners(lv, gp, p, g, idx, w);
+    // gradient of the encoding: slot 2i + k of level 4i + g is d_enc[i / 2][2 (i % 2) + k]
+    if (valid) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const float d0 = valid ? d_enc[j >> 1][2 * (j & 1)] : 0.0f;
-        const float d1 = valid ? d_enc[j >> 1][2 * (j & 1) + 1] : 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; c++) scatter_run(g_pos, idx[j][c], w[j][c] * d0, w[j][c] * d1, col, valid);
-      }
+      for (int i = 0; i < 4; i++)
+        d_feat[(4 * i + g) * cap + (j - j0)] = make_float2(d_enc[i >> 1][2 * (i & 1)], d_enc[i >> 1][2 * (i & 1) + 1]);
     }
     // density MLP weight gradients (activations as the forward's B slots)
     float h[16];
@@ -1065,11 +1119,21 @@ void diff_backward(Renderer& r, const float* d_rgb, float* g_pos, float* g_base,
                      D.ray_out.as<float4>(), d_rgb, D.d_out4.as<float4>());
   FVC_HIP(hipGetLastError());
   if (D.n_r > 0) {
-    hipLaunchKernelGGL(k_diff_net_bwd, dim3(bwd_blocks(D.n_r)), dim3(64 * BWD_WAVES), 0, s, (int)D.n_r,
-                       D.cached ? D.list_r.as<int>() : nullptr, D.s_pos.as<float>(), D.s_ray.as<int>(),
-                       D.rays.as<RayState>(), D.pos, m.grid, D.frags.as<float>(), D.d_out4.as<float4>(), g_pos,
-                       g_base, g_head);
-    FVC_HIP(hipGetLastError());
+    // the encoding's gradients pass through memory in chunks (at most 512 MiB)
+    const int64_t cap = std::min<int64_t>(D.n_r, (int64_t)1 << 22);
+    D.d_enc.ensure((size_t)cap * 16 * sizeof(float2));
+    const int* list = D.cached ? D.list_r.as<int>() : nullptr;
+    for (int64_t j0 = 0; j0 < D.n_r; j0 += cap) {
+      const int64_t nc = std::min<int64_t>(cap, D.n_r - j0);
+      hipLaunchKernelGGL(k_diff_net_bwd, dim3(bwd_blocks(nc)), dim3(64 * BWD_WAVES), 0, s, (int)j0, (int)(j0 + nc),
+                         list, D.s_pos.as<float>(), D.s_ray.as<int>(), D.rays.as<RayState>(), D.pos, m.grid,
+                         D.frags.as<float>(), D.d_out4.as<float4>(), D.d_enc.as<float2>(), cap, g_base, g_head);
+      FVC_HIP(hipGetLastError());
+      const int64_t per_block = 4 * 16 * SCATTER_SEG;
+      hipLaunchKernelGGL(k_diff_scatter, dim3((unsigned)(16 * ((nc + per_block - 1) / per_block))), dim3(256), 0, s,
+                         (int)j0, (int)(j0 + nc), list, D.s_pos.as<float>(), m.grid, D.d_enc.as<float>(), cap, g_pos);
+      FVC_HIP(hipGetLastError());
+    }
   }
   if (D.n_c > 0) {
     hipLaunchKernelGGL(k_diffc_head_bwd, dim3(2 * bwd_blocks(D.n_c)), dim3(64 * BWD_WAVES), 0, s, (int)D.n_c,
