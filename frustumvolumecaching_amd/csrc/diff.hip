@@ -528,17 +528,21 @@ struct KHead {
 // index arithmetic); the levels rotate over the blocks so that each XCD gets
 // coarse and fine ones.
 static const int SCATTER_SEG = 32;
+struct LevelList {
+  int n;
+  int l[MAX_LEVELS];
+};
 __global__ __launch_bounds__(256) void k_diff_scatter(int j0, int n, const int* __restrict__ list,
-                                                      const float* __restrict__ s_pos, GridParams gp,
+                                                      const float* __restrict__ s_pos, GridParams gp, LevelList ll,
                                                       const float* __restrict__ d_enc, int64_t cap,
                                                       float* __restrict__ g_pos) {
-  const int blk = blockIdx.x;
-  const int l = ((blk & 15) + (blk >> 4)) & 15;
+  const int grp = blockIdx.x / ll.n;
+  const int l = ll.l[(blockIdx.x + grp) % ll.n];
   const GridLevel L = gp.lv[l];
   const bool dense = (gp.dense_mask >> l) & 1u;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int xc = (lane >> 1) & 1, f = lane & 1;
-  const int64_t seg = ((int64_t)(blk >> 4) * 4 + wave) * 16 + (lane >> 2);
+  const int64_t seg = ((int64_t)grp * 4 + wave) * 16 + (lane >> 2);
   const int64_t first = j0 + seg * SCATTER_SEG;
   const int cnt = (int)(first >= n ? 0 : (n - first < SCATTER_SEG ? n - first : SCATTER_SEG));
   const float* de = d_enc + 2 * ((int64_t)l * cap) + f;
@@ -596,6 +600,205 @@ __global__ __launch_bounds__(256) void k_diff_scatter(int j0, int n, const int* 
     }
   }
   flush();
+}
+
+// Table gradient of the hashed levels without global atomics, in two kernels
+// over a chunk of samples.  k_diff_bin walks runs of BIN_SEG consecutive
+// samples per thread as k_diff_scatter does and turns each finished cell row
+// (y, z) into a record: the entries of corners x and x + 1 and the four sums
+// to add there.  Records are collected in LDS and written out sorted by
+// table slice of BIN_ENTRIES entries (one counter request per slice and
+// flush).  k_diff_bin_add gives each slice to one block, which sums its
+// records in LDS and adds the slice to the gradient with plain loads and
+// stores.  Entries x and x + 1 differ in the bits below the carry only
+// (res < BIN_ENTRIES), so a record has one slice.  LDS sums are FP64: on
+// gfx950 ds_add_f64 takes 26 cycles for a wave's random addresses,
+// ds_add_f32 185.
+//
+// Bound by the records' traffic (40 bytes each, written and read) in the
+// place of one 21 G/s atomic request per row: measured at 2^18 rays (14 M
+// samples, T 2^19), the table gradient 21.1 ms with k_diff_scatter alone, 9.2
+// ms with the 11 hashed levels in slices (4.5 + 2.6 ms here, 2.0 ms for the
+// dense levels in k_diff_scatter).
+// A slice holds `cap` records of a chunk; what does not fit (rays that
+// crowd into few cells) is added with atomics.
+static const int BIN_ENTRIES = 8192, BIN_SEG = 16, BIN_THREADS = 256;
+static const int BIN_BUF = 3072;                 // records buffered per block
+static const int BIN_MAX = 256;                  // slices of a level
+struct BinLevels {
+  int n;
+  int l[MAX_LEVELS], n_bins[MAX_LEVELS], first[MAX_LEVELS];  // first: the level's first slice
+};
+__global__ __launch_bounds__(BIN_THREADS) void k_diff_bin(int64_t j0, int n, int64_t d_off,
+                                                          const int* __restrict__ list,
+                                                          const float* __restrict__ s_pos, GridParams gp,
+                                                          BinLevels bl, const float2* __restrict__ d_enc,
+                                                          int64_t d_cap, int cap, int* __restrict__ cursor,
+                                                          float4* __restrict__ rec_val,
+                                                          uint32_t* __restrict__ rec_key,
+                                                          float* __restrict__ g_pos) {
+  __shared__ float4 s_val[BIN_BUF];
+  __shared__ uint32_t s_key[BIN_BUF];   // entry of corner x, trailing ones of x above bit 24
+  __shared__ int s_hist[BIN_MAX], s_base[BIN_MAX];
+  __shared__ int s_cnt;
+  const int li = blockIdx.x % bl.n, grp = blockIdx.x / bl.n;
+  const int l = bl.l[li], n_bins = bl.n_bins[li], bin0 = bl.first[li];
+  const GridLevel L = gp.lv[l];
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) s_cnt = 0;
+  const int64_t first = ((int64_t)grp * BIN_THREADS + threadIdx.x) * BIN_SEG;  // in the chunk
+  const int cnt = (int)(first >= n ? 0 : (n - first < BIN_SEG ? n - first : BIN_SEG));
+  const float2* de = d_enc + (int64_t)l * d_cap + d_off;
+  uint32_t cx = 0u, cy = 0u, cz = 0u;
+  float4 acc[4];  // row r: (x, feature 0), (x, 1), (x + 1, 0), (x + 1, 1)
+#pragma unroll
+  for (int r = 0; r < 4; r++) acc[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  auto entry = [&](uint32_t x, uint32_t y, uint32_t z) {
+    return (x ^ (y * 2654435761u) ^ (z * 805459861u)) & (L.size - 1u);
+  };
+  auto other = [&](uint32_t i0, uint32_t ones) { return (i0 ^ ((2u << ones) - 1u)) & (L.size - 1u); };
+  // sorts the buffered records by slice and writes them out
+  auto flush = [&](int c) {
+    for (int b = threadIdx.x; b < n_bins; b += BIN_THREADS) s_hist[b] = 0;
+    __syncthreads();
+    int rank[BIN_BUF / BIN_THREADS];
+#pragma unroll
+    for (int u = 0; u < BIN_BUF / BIN_THREADS; u++) {
+      const int i = u * BIN_THREADS + threadIdx.x;
+      if (i < c) rank[u] = atomicAdd(&s_hist[(s_key[i] & 0xffffffu) / BIN_ENTRIES], 1);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < n_bins; b += BIN_THREADS)
+      s_base[b] = s_hist[b] > 0 ? atomicAdd(&cursor[bin0 + b], s_hist[b]) : 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BIN_BUF / BIN_THREADS; u++) {
+      const int i = u * BIN_THREADS + threadIdx.x;
+      if (i >= c) break;
+      const uint32_t k = s_key[i], i0 = k & 0xffffffu, i1 = other(i0, k >> 24);
+      const int b = (int)(i0 / BIN_ENTRIES), at = s_base[b] + rank[u];
+      const float4 v = s_val[i];
+      if (at < cap) {
+        const int64_t q = (int64_t)(bin0 + b) * cap + at;
+        rec_val[q] = v;
+        rec_key[q] = (i0 & (BIN_ENTRIES - 1u)) | ((i1 & (BIN_ENTRIES - 1u)) << 16);
+      } else {
+        float* g0 = g_pos + 2 * ((size_t)L.offset + i0);
+        float* g1 = g_pos + 2 * ((size_t)L.offset + i1);
+        unsafeAtomicAdd(g0, v.x);
+        unsafeAtomicAdd(g0 + 1, v.y);
+        unsafeAtomicAdd(g1, v.z);
+        unsafeAtomicAdd(g1 + 1, v.w);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) s_cnt = 0;
+    __syncthreads();
+  };
+  __syncthreads();
+  for (int k = 0; k <= BIN_SEG; k++) {
+    const bool in = k < cnt;
+    float2 d = make_float2(0.0f, 0.0f);
+    uint32_t gx = 0u, gy = 0u, gz = 0u;
+    float wx = 0.0f, wy = 0.0f, wz = 0.0f;
+    if (in) {
+      const int64_t j = j0 + first + k;
+      const int64_t sl = list ? list[j] : j;
+      const float px = fminf_(fmaxf_(s_pos[3 * sl], 0.0f), 1.0f);
+      const float py = fminf_(fmaxf_(s_pos[3 * sl + 1], 0.0f), 1.0f);
+      const float pz = fminf_(fmaxf_(s_pos[3 * sl + 2], 0.0f), 1.0f);
+      d = de[first + k];
+      const float ax = px * L.scale + 0.5f, ay = py * L.scale + 0.5f, az = pz * L.scale + 0.5f;
+      const float fx = floorf(ax), fy = floorf(ay), fz = floorf(az);
+      gx = (uint32_t)(int)fx; gy = (uint32_t)(int)fy; gz = (uint32_t)(int)fz;
+      wx = ax - fx; wy = ay - fy; wz = az - fz;
+    }
+    // a finished cell with something to add becomes four records
+    bool emit = !in || gx != cx || gy != cy || gz != cz;
+    if (emit) {
+      bool any = false;
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        any = any || acc[r].x != 0.0f || acc[r].y != 0.0f || acc[r].z != 0.0f || acc[r].w != 0.0f;
+      emit = any;
+    }
+    const unsigned long long m = __ballot(emit);
+    const int ne = __popcll(m);
+    int base = 0;
+    if (lane == 0 && ne > 0) base = atomicAdd(&s_cnt, 4 * ne);
+    base = __shfl(base, 0, 64);
+    if (emit) {
+      const int at = base + __popcll(m & ((1ull << lane) - 1ull));
+      const uint32_t ones = (uint32_t)__builtin_ctz(~cx);  // x < 2^24
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        s_val[at + r * ne] = acc[r];
+        s_key[at + r * ne] = entry(cx, cy + (r & 1), cz + (r >> 1)) | (ones << 24);
+      }
+    }
+    if (!in || gx != cx || gy != cy || gz != cz) {
+      cx = gx; cy = gy; cz = gz;
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    const float ux = 1.0f - wx, uy = 1.0f - wy, uz = 1.0f - wz;
+    const float wxy[4] = {ux * uy, wx * uy, ux * wy, wx * wy};
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float w = (r & 2) ? wz : uz, w0 = wxy[2 * (r & 1)] * w, w1 = wxy[2 * (r & 1) + 1] * w;
+      acc[r].x = acc[r].x + w0 * d.x;
+      acc[r].y = acc[r].y + w0 * d.y;
+      acc[r].z = acc[r].z + w1 * d.x;
+      acc[r].w = acc[r].w + w1 * d.y;
+    }
+    __syncthreads();
+    const int c = s_cnt;
+    __syncthreads();
+    // a step adds at most 4 records a thread
+    if (c > BIN_BUF - 4 * BIN_THREADS || (k == BIN_SEG && c > 0)) flush(c);
+  }
+}
+
+__global__ void k_diff_zero(int* __restrict__ p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+// one slice of one level: its records summed in LDS, then added to the
+// gradient (the block is the only one that touches these entries)
+__global__ __launch_bounds__(1024) void k_diff_bin_add(GridParams gp, BinLevels bl, int cap,
+                                                       int* __restrict__ cursor,
+                                                       const float4* __restrict__ rec_val,
+                                                       const uint32_t* __restrict__ rec_key,
+                                                       float* __restrict__ g_pos) {
+  __shared__ double acc[2 * BIN_ENTRIES];
+  // the finest levels, with the most records, first
+  int li = bl.n - 1, b = blockIdx.x;
+  while (b >= bl.n_bins[li]) b -= bl.n_bins[li--];
+  const GridLevel L = gp.lv[bl.l[li]];
+  const int bin = bl.first[li] + b;
+  const int c = min(cursor[bin], cap);
+  if (c <= 0) return;
+  const int n_ent = min((int)L.size - b * BIN_ENTRIES, BIN_ENTRIES);
+  for (int i = threadIdx.x; i < 2 * n_ent; i += 1024) acc[i] = 0.0;
+  __syncthreads();
+  if (threadIdx.x == 0) cursor[bin] = 0;  // for the next chunk
+  const float4* rv = rec_val + (int64_t)bin * cap;
+  const uint32_t* rk = rec_key + (int64_t)bin * cap;
+  for (int i = threadIdx.x; i < c; i += 1024) {
+    const uint32_t k = rk[i];
+    const float4 v = rv[i];
+    double* a0 = acc + 2 * (k & 0xffffu);
+    double* a1 = acc + 2 * (k >> 16);
+    unsafeAtomicAdd(a0, (double)v.x);
+    unsafeAtomicAdd(a0 + 1, (double)v.y);
+    unsafeAtomicAdd(a1, (double)v.z);
+    unsafeAtomicAdd(a1 + 1, (double)v.w);
+  }
+  __syncthreads();
+  float* g = g_pos + 2 * ((size_t)L.offset + (size_t)b * BIN_ENTRIES);
+  for (int i = threadIdx.x; i < 2 * n_ent; i += 1024)
+    if (acc[i] != 0.0) g[i] = g[i] + (float)acc[i];
 }
 
 // colour MLP backward of a tile: d_o (output rows 4g..4g+3), d_z1
@@ -1000,6 +1203,59 @@ static int64_t scan_counts(DiffState& D, int* counts, int64_t* offs, int n, hipS
   return total;
 }
 
+// the encoding's gradients of samples [j0, j0 + n) into the table's gradient:
+// hashed levels through the slice bins, the others (and all of a small
+// batch) with atomics.  Bins pay for reading and writing every slice once
+// per chunk: measured at T 2^19 (16 to 140 thousand samples) the two are equal at 35 to
+// 65 thousand, below that atomics are ahead.
+// Levels of more than BIN_MAX slices (T > 2^21) would fill a slice's place in
+// a flush with less than a cache line.
+static const int64_t BIN_MIN_SAMPLES = 1 << 16, BIN_CHUNK = 1 << 19;
+static void scatter_table(DiffState& D, const GridParams& gp, const int* list, int64_t j0, int64_t n, int64_t d_cap,
+                          float* g_pos, hipStream_t s) {
+  LevelList ll{};
+  BinLevels bl{};
+  int n_bins = 0, most = 1;
+  for (int l = 0; l < gp.n_levels; l++) {
+    const GridLevel& L = gp.lv[l];
+    const int nb = (int)((L.size + BIN_ENTRIES - 1) / BIN_ENTRIES);
+    if (n < BIN_MIN_SAMPLES || ((gp.dense_mask >> l) & 1u) || nb > BIN_MAX || L.res >= (uint32_t)BIN_ENTRIES) {
+      ll.l[ll.n++] = l;
+      continue;
+    }
+    bl.l[bl.n] = l;
+    bl.n_bins[bl.n] = nb;
+    bl.first[bl.n++] = n_bins;
+    n_bins += nb;
+    most = std::max(most, nb);
+  }
+  if (ll.n > 0) {
+    const int64_t per_block = 4 * 16 * SCATTER_SEG;
+    hipLaunchKernelGGL(k_diff_scatter, dim3((unsigned)(ll.n * ((n + per_block - 1) / per_block))), dim3(256), 0, s,
+                       (int)j0, (int)(j0 + n), list, D.s_pos.as<float>(), gp, ll, D.d_enc.as<float>(), d_cap, g_pos);
+    FVC_HIP(hipGetLastError());
+  }
+  if (bl.n == 0) return;
+  // room for a quarter more than an even spread of four records a sample
+  const int64_t chunk = std::min<int64_t>(n, BIN_CHUNK);
+  const int cap = (int)(5 * chunk / most + 1024);
+  D.bin_cursor.ensure((size_t)n_bins * sizeof(int));
+  D.bin_val.ensure((size_t)n_bins * cap * sizeof(float4));
+  D.bin_key.ensure((size_t)n_bins * cap * sizeof(uint32_t));
+  hipLaunchKernelGGL(k_diff_zero, dim3((n_bins + 255) / 256), dim3(256), 0, s, D.bin_cursor.as<int>(), n_bins);
+  for (int64_t c0 = 0; c0 < n; c0 += chunk) {
+    const int64_t nc = std::min<int64_t>(chunk, n - c0);
+    const int64_t per_block = (int64_t)BIN_THREADS * BIN_SEG;
+    hipLaunchKernelGGL(k_diff_bin, dim3((unsigned)(bl.n * ((nc + per_block - 1) / per_block))), dim3(BIN_THREADS), 0, s,
+                       j0 + c0, (int)nc, c0, list, D.s_pos.as<float>(), gp, bl, D.d_enc.as<float2>(), d_cap, cap,
+                       D.bin_cursor.as<int>(), D.bin_val.as<float4>(), D.bin_key.as<uint32_t>(), g_pos);
+    FVC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_diff_bin_add, dim3(n_bins), dim3(1024), 0, s, gp, bl, cap, D.bin_cursor.as<int>(),
+                       D.bin_val.as<float4>(), D.bin_key.as<uint32_t>(), g_pos);
+    FVC_HIP(hipGetLastError());
+  }
+}
+
 void diff_forward(Renderer& r, const fvc_raymarch_info& rm, const int* pix, int n, const float* pos,
                   const float* base, const float* head, float* rgb, fvc_diff_stats* stats, bool cached) {
   const Model& m = *r.model;
@@ -1129,10 +1385,7 @@ void diff_backward(Renderer& r, const float* d_rgb, float* g_pos, float* g_base,
                          list, D.s_pos.as<float>(), D.s_ray.as<int>(), D.rays.as<RayState>(), D.pos, m.grid,
                          D.frags.as<float>(), D.d_out4.as<float4>(), D.d_enc.as<float2>(), cap, g_base, g_head);
       FVC_HIP(hipGetLastError());
-      const int64_t per_block = 4 * 16 * SCATTER_SEG;
-      hipLaunchKernelGGL(k_diff_scatter, dim3((unsigned)(16 * ((nc + per_block - 1) / per_block))), dim3(256), 0, s,
-                         (int)j0, (int)(j0 + nc), list, D.s_pos.as<float>(), m.grid, D.d_enc.as<float>(), cap, g_pos);
-      FVC_HIP(hipGetLastError());
+      scatter_table(D, m.grid, list, j0, nc, cap, g_pos, s);
     }
   }
   if (D.n_c > 0) {

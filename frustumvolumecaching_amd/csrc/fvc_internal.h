@@ -346,6 +346,7 @@ struct DiffState {
   DevBuf frag_index, frags;        // FP32 MFMA fragments of the caller's weights
   DevBuf rays, counts, offsets, ray_out, n_walk, scan_tmp;
   DevBuf s_pos, s_dt, s_ray, out4, d_out4;
+  DevBuf bin_cursor, bin_val, bin_key;  // backward: records per table slice
   DevBuf d_enc;  // backward: gradients of the encoding, [16 levels][chunk of samples] float2
   DevBuf counts_c, off_r, off_c, counts_all, list_r, list_c;  // cached mode
   int n = 0;
