@@ -1130,6 +1130,42 @@ __global__ __launch_bounds__(256) void k_diffc_head_fwd(int n, const int* __rest
   }
 }
 
+// Voxel gradients of a tile of 16 samples.  Bound by atomic requests (21 G/s;
+// the lanes of an instruction within one 64-byte line are one request): lane
+// (2 y + x) * 9 + k takes value k (8 latents, density) of corner column
+// (x, y), so a voxel's nine words, and its x neighbour's, go in one
+// instruction; and a ray's next sample is usually one froxel further in z,
+// so the sum for corner z + 1 waits for the next sample's corner z.
+// Measured at 65521 rays (3.8 M cache samples) against one atomic per corner
+// and value, a corner's values in one lane: k_diffc_head_bwd 11.3 -> 1.2 ms.
+static const uint32_t NO_VOXEL = 0xffffffffu;  // outside the frustum or unset; indices stay below
+struct PoolTile {
+  uint32_t v[16][2][4];   // voxel in the order of g_pool [sample][z][2 x + y]
+  float wl[16][2][4], wd[16][2][4];
+  float d[16][9];
+};
+__device__ __forceinline__ void scatter_pool(const PoolTile& pt, int lane, float* __restrict__ g_pool) {
+  if (lane >= 36) return;
+  const int k = lane % 9, c = lane / 9, g = 2 * (c & 1) + (c >> 1);
+  auto add = [&](uint32_t v, float x) {
+    if (v != NO_VOXEL && x != 0.0f) unsafeAtomicAdd(&g_pool[(size_t)v * 10 + k], x);
+  };
+  uint32_t pv = NO_VOXEL;
+  float pend = 0.0f;
+  for (int s = 0; s < 16; s++) {
+    const uint32_t v0 = pt.v[s][0][g], v1 = pt.v[s][1][g];
+    const float d = pt.d[s][k];
+    float x0 = (k < 8 ? pt.wl[s][0][g] : pt.wd[s][0][g]) * d;
+    const float x1 = (k < 8 ? pt.wl[s][1][g] : pt.wd[s][1][g]) * d;
+    if (v0 == pv) x0 = x0 + pend;
+    else add(pv, pend);
+    add(v0, x0);
+    pv = v1;
+    pend = x1;
+  }
+  add(pv, pend);
+}
+
 __global__ __launch_bounds__(64 * BWD_WAVES) void k_diffc_head_bwd(int n, const int* __restrict__ list,
                                                         const float* __restrict__ s_pos,
                                                         const int* __restrict__ s_ray,
@@ -1158,22 +1194,25 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_diffc_head_bwd(int n, const 
     f4 d_o, d_z1[4], d_xh;
     head_backward<F_H1>(fr, lane, g, a, dq, d_o, d_z1, d_xh);
     head_wgrad(stage, a, d_o, d_z1, wave, col, g, acc_h);
-    // dL/dl_i of latent i (row i + 1: lane group (i + 1) / 4, element (i + 1) % 4)
-    float d_lat[8];
+    // the tile's corner voxels, their weights and the samples' gradients
+    // (dL/dl_i of latent i is row i + 1 of d_xh), then the scatter
+    static_assert(BWD_WAVES * sizeof(PoolTile) <= sizeof(stage), "the tiles share the staging rows");
+    PoolTile* pt = reinterpret_cast<PoolTile*>(stage) + wave;
 #pragma unroll
-    for (int i = 0; i < 8; i++) d_lat[i] = __shfl(d_xh[(i + 1) & 3], col + 16 * ((i + 1) >> 2), 64);
-    const float d_dsum = L.dsum > 1e-6f ? dq.w / L.dsum : 0.0f;
-    if (valid) {
-#pragma unroll
-      for (int cc = 0; cc < 2; cc++) {
-        if (L.v[cc] < 0) continue;
-        float* gv = g_pool + L.v[cc] * 10;
-        const float wl = L.w[cc] / L.wsum;
-#pragma unroll
-        for (int i = 0; i < 8; i++) unsafeAtomicAdd(&gv[i], wl * d_lat[i]);
-        unsafeAtomicAdd(&gv[8], L.w[cc] * d_dsum);
-      }
+    for (int cc = 0; cc < 2; cc++) {
+      pt->v[col][cc][g] = valid && L.v[cc] >= 0 ? (uint32_t)L.v[cc] : NO_VOXEL;
+      pt->wl[col][cc][g] = L.w[cc] / L.wsum;
+      pt->wd[col][cc][g] = L.w[cc];
     }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = 4 * g + e;
+      if (r >= 1 && r <= 8) pt->d[col][r - 1] = d_xh[e];
+    }
+    if (g == 0) pt->d[col][8] = L.dsum > 1e-6f ? dq.w / L.dsum : 0.0f;
+    wave_sync();
+    scatter_pool(*pt, lane, g_pool);
+    __syncthreads();  // the staging rows are free again
   }
   flush_head(g_head, wave, col, g, acc_h);
 }
