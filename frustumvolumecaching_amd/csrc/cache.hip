@@ -772,14 +772,20 @@ __global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int 
                                                      int8_t* __restrict__ dbg_codes, int dbg_k,
                                                      int* __restrict__ dbg_n) {
   const int n_alive = ctl[CTL_ALIVE + par];
-  if ((int)(blockIdx.x * blockDim.x) >= n_alive) return;  // whole block past the alive rays
+  const int G = mg.tab.n_rows > 0 ? group_lanes(n_alive) : 1;
+  const bool group = G > 1;
+  const int rays_per_block = 256 / G;
+  if ((int)blockIdx.x * rays_per_block >= n_alive) return;  // whole block past the alive rays
   const int n_steps = ctl[CTL_NSTEPS];
   int* cnt_r = ctl + CTL_R;
   int* cnt_c = ctl + CTL_C;
   int* step_counter = ctl + CTL_BINS;
-  __shared__ uint32_t coarse[16 * COARSE_WORDS];
+  extern __shared__ uint32_t coarse[];  // march_lds
   load_coarse(coarse_g, mg.occ.nlvl, coarse);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
+  const int sub = threadIdx.x & (G - 1);
+  // group: the ray's samples
+  float* ts = reinterpret_cast<float*>(coarse + mg.occ.nlvl * COARSE_WORDS) + (threadIdx.x / G) * MAX_STEPS_PER_LAUNCH;
   const bool valid = i < n_alive;
   int cnt = 0, bins = 0;
   uint64_t res_mask = 0, cache_mask = 0;  // class of march sample k
@@ -793,7 +799,7 @@ __global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int 
     r = rconst[px];
     r.t = dy.t;
     r.j = dy.j;
-    if (r.j == 0) {
+    if (r.j == 0 && sub == 0) {
       // first launch of the ray: its per-pixel tables (the colour MLP's SH
       // input depends on the direction only; split models also read the ray)
       uint4 lo, hi;
@@ -808,15 +814,21 @@ __global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int 
     }
     alive = true;
     MarchRay mr = march_ray(r, mg.tab);
-    int trips = 0;
-    while (cnt < n_steps && trips < trip_cutoff) {
-      trips++;
-      float t0;
-      const int res = march_trip(mg, coarse, mr, t0, bins);
-      if (res == TRIP_END) { alive = false; break; }
-      if (res == TRIP_SAMPLE) {
-        t_scr[(int64_t)cnt * n_alive + i] = t0;
-        cnt++;
+    if (group && group_usable(mg, mr)) {
+      alive = G == 16 ? march_group<16>(mg, coarse, mr, n_steps, ts, cnt, bins)
+                      : march_group<4>(mg, coarse, mr, n_steps, ts, cnt, bins);
+    } else {
+      int trips = 0;
+      while (cnt < n_steps && trips < trip_cutoff) {
+        trips++;
+        float t0;
+        const int res = march_trip(mg, coarse, mr, t0, bins);
+        if (res == TRIP_END) { alive = false; break; }
+        if (res == TRIP_SAMPLE) {
+          if (group) ts[cnt] = t0;
+          else t_scr[(int64_t)cnt * n_alive + i] = t0;
+          cnt++;
+        }
       }
     }
     r.t = mr.t1;
@@ -824,13 +836,30 @@ __global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int 
     // classification (sample_cache_performance_kernel, cache_performance_renderer.cu:96-160)
     oc = transform(cv.cam.world2cam, mr.o.x, mr.o.y, mr.o.z, 1.0f);
     dc = transform(cv.cam.world2cam, mr.d.x, mr.d.y, mr.d.z, 0.0f);
-    // CLS samples per step; each step issues all its loads (t0, known range,
-    // brick slot, then voxel density) before using them, from clamped
-    // addresses whose results are selected away where they do not apply
+    // one lane per ray: CLS samples per step; each step issues all its loads
+    // (t0, known range, brick slot, then voxel density) before using them, from
+    // clamped addresses whose results are selected away where they do not
+    // apply.  Groups: one sample per lane.
     constexpr int CLS = 4;
     const float* dens = cv.lat8 ? &cv.pool8[0].density : &cv.pool[0].density;
     const int vstride = cv.lat8 ? (int)(sizeof(Voxel8) / 4) : (int)(sizeof(Voxel) / 4);
-    for (int k0 = 0; k0 < cnt; k0 += CLS) {
+    const uint64_t keep_r = render_mode != FVC_RENDER_ONLY_CACHE ? ~0ull : 0ull;
+    const uint64_t keep_c = render_mode != FVC_RENDER_ONLY_RESAMPLED ? ~0ull : 0ull;
+    if (group) {
+      wave_sync();  // the samples in LDS
+      const int sh = lane_id() & ~(G - 1);
+      for (int k0 = 0; k0 < cnt; k0 += G) {
+        const float t0 = ts[min(k0 + sub, cnt - 1)];
+        const int cls = classify_sample(cv, oc, dc, t0, step_dt(mg.st, t0));
+        const bool in = k0 + sub < cnt;
+        const uint64_t all = (1ull << G) - 1ull;
+        res_mask |= ((__ballot(in && cls == SAMPLE_RESAMPLE) >> sh) & all) << k0;
+        cache_mask |= ((__ballot(in && cls == SAMPLE_CACHE) >> sh) & all) << k0;
+      }
+      res_mask &= keep_r;
+      cache_mask &= keep_c;
+    }
+    for (int k0 = 0; k0 < (group ? 0 : cnt); k0 += CLS) {
       float t0v[CLS], tf[CLS], known[CLS], dv[CLS];
       V3 f[CLS];
       bool in_fov[CLS], inside[CLS];
@@ -871,46 +900,68 @@ __global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int 
   }
   const int nr = __popcll(res_mask), nc = __popcll(cache_mask);
   int slot[3];
-  block_reserve<3>({nr, nc, bins}, {cnt_r, cnt_c, step_counter}, slot);
-  const int off_r = slot[0], off_c = slot[1];
+  block_reserve<3>({sub == 0 ? nr : 0, sub == 0 ? nc : 0, sub == 0 ? bins : 0}, {cnt_r, cnt_c, step_counter}, slot);
+  const int off_r = group ? __shfl(slot[0], 0, G) : slot[0], off_c = group ? __shfl(slot[1], 0, G) : slot[1];
   if (valid) {
     const V3 o = {r.ox, r.oy, r.oz}, d = {r.dx, r.dy, r.dz};
     const float pxf = __builtin_bit_cast(float, px);
     uint64_t order = 0;  // bit q set: the q-th kept sample is a cache sample
-    int kr = 0, kc = 0;
     const uint64_t kept = res_mask | cache_mask;
-    for (int k0 = 0; k0 < cnt; k0 += CLS_EMIT) {
-      if (((kept >> k0) & ((1ull << CLS_EMIT) - 1ull)) == 0ull) continue;
-      float t0v[CLS_EMIT];
-#pragma unroll
-      for (int u = 0; u < CLS_EMIT; u++) t0v[u] = t_scr[(int64_t)min(k0 + u, cnt - 1) * n_alive + i];
-#pragma unroll
-      for (int u = 0; u < CLS_EMIT; u++) {
-        const int k = k0 + u;
-        if (k >= cnt) break;
-        const bool is_r = (res_mask >> k) & 1ull, is_c = (cache_mask >> k) & 1ull;
-        if (!is_r && !is_c) continue;
-        const float t0 = t0v[u];
-        const float tm2 = t0 + step_dt(mg.st, t0) * 0.5f;
-        if (is_r) {
-          // generateNetworkInput_resample_perf_kernel (198-240): t_mid = t0 + dt/2
-          const V3 p = contract(o + tm2 * d, con);
-          const int64_t q = (int64_t)off_r + kr;
-          s_pos[q] = make_float4(p.x, p.y, p.z, pxf);
-          s_t0[q] = t0;
-        } else {
-          // generateNetworkInput_preparation_perf_kernel (242-313)
-          float tf;
-          const V3 f = cam2froxel(oc + tm2 * dc, cv.cam, cv.st, tf);
-          const int64_t q = (int64_t)off_c + kc;
-          c_rec[q] = make_float4(f.x, f.y, f.z, __builtin_bit_cast(float, px));
-          c_t0[q] = t0;
+    // writes resample sample kr of the ray
+    auto emit_r = [&](float t0, int kr) {
+      // generateNetworkInput_resample_perf_kernel (198-240): t_mid = t0 + dt/2
+      const float tm2 = t0 + step_dt(mg.st, t0) * 0.5f;
+      const V3 p = contract(o + tm2 * d, con);
+      const int64_t q = (int64_t)off_r + kr;
+      s_pos[q] = make_float4(p.x, p.y, p.z, pxf);
+      s_t0[q] = t0;
+    };
+    // writes cache sample kc of the ray
+    auto emit_c = [&](float t0, int kc) {
+      // generateNetworkInput_preparation_perf_kernel (242-313)
+      const float tm2 = t0 + step_dt(mg.st, t0) * 0.5f;
+      float tf;
+      const V3 f = cam2froxel(oc + tm2 * dc, cv.cam, cv.st, tf);
+      const int64_t q = (int64_t)off_c + kc;
+      c_rec[q] = make_float4(f.x, f.y, f.z, pxf);
+      c_t0[q] = t0;
+    };
+    if (group) {
+      for (int k = sub; k < cnt; k += G) {
+        const uint64_t below = (1ull << k) - 1ull;
+        const int kr = __popcll(res_mask & below), kc = __popcll(cache_mask & below);
+        if ((res_mask >> k) & 1ull) emit_r(ts[k], kr);
+        else if ((cache_mask >> k) & 1ull) {
+          emit_c(ts[k], kc);
           order |= 1ull << (kr + kc);
         }
-        kr += is_r ? 1 : 0;
-        kc += is_c ? 1 : 0;
+      }
+      for (int m = 1; m < G; m <<= 1) order |= __shfl_xor(order, m, G);
+    } else {
+      int kr = 0, kc = 0;
+      for (int k0 = 0; k0 < cnt; k0 += CLS_EMIT) {
+        if (((kept >> k0) & ((1ull << CLS_EMIT) - 1ull)) == 0ull) continue;
+        float t0v[CLS_EMIT];
+#pragma unroll
+        for (int u = 0; u < CLS_EMIT; u++) t0v[u] = t_scr[(int64_t)min(k0 + u, cnt - 1) * n_alive + i];
+#pragma unroll
+        for (int u = 0; u < CLS_EMIT; u++) {
+          const int k = k0 + u;
+          if (k >= cnt) break;
+          const bool is_r = (res_mask >> k) & 1ull, is_c = (cache_mask >> k) & 1ull;
+          if (!is_r && !is_c) continue;
+          if (is_r) {
+            emit_r(t0v[u], kr);
+          } else {
+            emit_c(t0v[u], kc);
+            order |= 1ull << (kr + kc);
+          }
+          kr += is_r ? 1 : 0;
+          kc += is_c ? 1 : 0;
+        }
       }
     }
+    if (sub != 0) return;
     rays[i] = RayDyn{r.t, r.j};
     entry[i] = make_int4(off_r, nr, off_c, nc);
     order_out[i] = order;
@@ -1326,9 +1377,13 @@ __global__ __launch_bounds__(256) void k_cache_composite(
   // dbg_comp (optional, inspection only): per pixel the resampled and cached
   // samples composited, up to and including the one that ends the ray
   const int n_alive = ctl[CTL_ALIVE + par];
-  if ((int)(blockIdx.x * blockDim.x) >= n_alive) return;
+  const int G = group_lanes(n_alive);
+  const bool group = G > 1;
+  const int rays_per_block = 256 / G;
+  if ((int)blockIdx.x * rays_per_block >= n_alive) return;
   int* counter = ctl + CTL_ALIVE + (par ^ 1);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
+  const int sub = threadIdx.x & (G - 1);
   const bool valid = i < n_alive;
   bool keep = false;
   int px = 0;
@@ -1345,7 +1400,17 @@ __global__ __launch_bounds__(256) void k_cache_composite(
     int kr = 0, kc = 0;
     int n_done = 0;       // samples composited
     // the two streams interleaved in march (= t0) order, batch by batch
-    for (int k0 = 0; k0 < n && visible; k0 += COMPOSITE_BATCH) {
+    for (int k0 = 0; group && k0 < n && visible; k0 += G) {
+      const int k = min(k0 + sub, n - 1);
+      const int before = __popcll(ord & ((1ull << k) - 1ull));  // cache samples before sample k
+      const bool from_cache = (ord >> k) & 1ull;
+      const int q = from_cache ? e.z + before : e.x + k - before;
+      const uint2 v = (from_cache ? c_out : s_out)[q];
+      const float t = (from_cache ? c_t0 : s_t0)[q];
+      visible = G == 16 ? composite_group<16>(res, v, t, n - k0, st, alpha_thre, n_done)
+                        : composite_group<4>(res, v, t, n - k0, st, alpha_thre, n_done);
+    }
+    for (int k0 = 0; !group && k0 < n && visible; k0 += COMPOSITE_BATCH) {
       uint2 v[COMPOSITE_BATCH];
       float t[COMPOSITE_BATCH];
 #pragma unroll
@@ -1366,9 +1431,9 @@ __global__ __launch_bounds__(256) void k_cache_composite(
           n_done++;
         }
     }
-    keep = visible && ray_alive != 0;
-    if (!keep) results[px] = res;
-    if (dbg_comp) {
+    keep = visible && ray_alive != 0 && sub == 0;
+    if (!keep && sub == 0) results[px] = res;
+    if (dbg_comp && sub == 0) {
       int cc = 0;
       for (int k = 0; k < n_done; k++) cc += (int)((ord >> k) & 1u);
       const int2 d = dbg_comp[px];
@@ -1416,7 +1481,7 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
   int* ctl = r.counters.as<int>();
   const int64_t target = std::min<int64_t>(vs.target(r.target_batch), cap - 64);
   const int64_t n_bound = std::min<int64_t>(cap - 64, (int64_t)n0 * r.max_steps);  // samples per launch
-  const dim3 grid((n0 + 255) / 256);
+  const dim3 grid(ray_blocks(n0));
   const int head_blocks = (int)std::min<int64_t>((n_bound + 255) / 256, 256 * 16);
   // loop trips per ray and launch; a performance knob only (a ray resumes
   // where it stopped), like the reference's step_cutoff
@@ -1429,7 +1494,7 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, target, r.max_steps, cap - 64, 0);
       Handles h;
       ev = P.begin(s);
-      hipLaunchKernelGGL(k_cache_march, grid, dim3(256), 0, s, ctl, cur, cutoff, mg, m.con, m.coarse.as<uint32_t>(), cv,
+      hipLaunchKernelGGL(k_cache_march, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl, cur, cutoff, mg, m.con, m.coarse.as<uint32_t>(), cv,
                          r.rays[cur].as<RayDyn>(), r.ray_entry.as<int4>(), r.ray_alive.as<int>(),
                          r.t_scratch.as<float>(), r.s_pos.as<float4>(), r.s_t0.as<float>(), r.c_rec.as<float4>(), r.c_t0.as<float>(), r.ray_pix[cur].as<int>(), r.ray_sh.as<uint4>(),
                          m.net.split_head ? r.ray_od.as<float4>() : nullptr,

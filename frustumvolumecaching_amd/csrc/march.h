@@ -357,4 +357,61 @@ FVC_HD int march_trip(const MarchGrid& g, const uint32_t* coarse, MarchRay& r, f
   return TRIP_EMPTY;
 }
 
+// ------------------------------------------------------------ lane groups
+// A ray marched by a group of G lanes (G <= 16): lane k tests bin j + k of the
+// ray's step-table row by itself (march_probe), the group's answers as bit
+// masks give the samples, the end of the ray or where to go on (group_plan),
+// and the empty box that reaches farthest is jumped over as in march_trip.
+// The samples are those of march_trip: a bin is one when its own midpoint is
+// occupied, and only bins inside a box found empty are jumped over.
+
+// The group's bins come from the table: the row must reach past far.
+FVC_HD bool group_usable(const MarchGrid& g, const MarchRay& r) {
+  if (r.row.base < 0 || r.row.last < 0) return false;
+  const float* e = g.tab.t + r.row.base + r.row.last;
+  return (e[0] + e[1]) * 0.5f > r.far_;
+}
+
+enum { PROBE_EMPTY = 0, PROBE_SAMPLE = 1, PROBE_PAST = 2 };
+// Bin j of the ray: its start t0, and, when it lies in an empty box, the
+// ray parameter hi up to which the box reaches (else a negative number).
+FVC_HD int march_probe(const MarchGrid& g, const uint32_t* coarse, const MarchRay& r, int j, float& t0, float& hi) {
+  t0 = 0.0f;
+  hi = -1.0f;
+  if (j > r.row.last) return PROBE_PAST;
+  const float* e = g.tab.t + r.row.base + j;
+  t0 = e[0];
+  const float tm = (t0 + e[1]) * 0.5f;
+  if (tm > r.far_) return PROBE_PAST;
+  Skip sk = no_skip();
+  if (occ_query(r.o + tm * r.d, g.occ, g.bf64, coarse, r.slab, sk)) return PROBE_SAMPLE;
+  if (in_skip(sk, tm)) hi = sk.hi;
+  return PROBE_EMPTY;
+}
+
+// What a group step comes to: the samples among its bins (at most budget, the
+// step ends right after the last one taken), how many bins it passes, and
+// whether the ray ended (a midpoint past far) or the budget is used up.
+struct GroupPlan {
+  uint32_t samples;
+  int bins;
+  bool ended, full;
+};
+FVC_HD GroupPlan group_plan(int G, uint32_t occ, uint32_t past, int budget) {
+  GroupPlan p;
+  const int n = past ? __builtin_ctz(past) : G;
+  p.samples = occ & ((1u << n) - 1u);
+  p.ended = n < G;
+  p.bins = n;
+  p.full = __builtin_popcount(p.samples) >= budget;
+  if (p.full) {
+    uint32_t rest = p.samples;
+    for (int k = 1; k < budget; k++) rest &= rest - 1u;
+    p.bins = __builtin_ctz(rest) + 1;
+    p.samples &= (2u << (p.bins - 1)) - 1u;
+    p.ended = false;
+  }
+  return p;
+}
+
 }  // namespace fvc

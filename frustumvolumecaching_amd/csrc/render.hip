@@ -69,13 +69,19 @@ __global__ __launch_bounds__(256) void k_march(int* __restrict__ ctl, int par, M
                                                float* __restrict__ t_scr, float4* __restrict__ s_pos,
                                                uint4* __restrict__ ray_sh, float* __restrict__ s_t0) {
   const int n_alive = ctl[CTL_ALIVE + par];
-  if ((int)(blockIdx.x * blockDim.x) >= n_alive) return;  // whole block past the alive rays
+  const int G = mg.tab.n_rows > 0 ? group_lanes(n_alive) : 1;
+  const bool group = G > 1;
+  const int rays_per_block = 256 / G;
+  if ((int)blockIdx.x * rays_per_block >= n_alive) return;  // whole block past the alive rays
   const int n_steps = ctl[CTL_NSTEPS];
   int* s_counter = ctl + CTL_R;
   int* step_counter = ctl + CTL_BINS;
-  __shared__ uint32_t coarse[16 * COARSE_WORDS];
+  extern __shared__ uint32_t coarse[];  // march_lds
   if constexpr (!MULTI) load_coarse(coarse_g, mg.occ.nlvl, coarse);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
+  const int sub = threadIdx.x & (G - 1);
+  // group: the ray's samples
+  float* ts = reinterpret_cast<float*>(coarse + mg.occ.nlvl * COARSE_WORDS) + (threadIdx.x / G) * MAX_STEPS_PER_LAUNCH;
   const bool valid = i < n_alive;
   int cnt = 0, bins = 0;
   bool alive = false;
@@ -87,7 +93,7 @@ __global__ __launch_bounds__(256) void k_march(int* __restrict__ ctl, int par, M
     rs = rconst[px];
     rs.t = dy.t;
     rs.j = dy.j;
-    if (rs.j == 0) {
+    if (rs.j == 0 && sub == 0) {
       // first launch of the ray: the colour MLP's SH input of its direction
       uint4 lo, hi;
       const V3 d01 = unit_to_01(V3{rs.dx, rs.dy, rs.dz});
@@ -106,45 +112,59 @@ __global__ __launch_bounds__(256) void k_march(int* __restrict__ ctl, int par, M
       cz = coarse;
     }
     MarchRay r = march_ray(rs, g.tab);
-    while (cnt < n_steps) {
-      float t0;
-      const int res = march_trip(g, cz, r, t0, bins);
-      if (res == TRIP_END) { alive = false; break; }
-      if (res == TRIP_SAMPLE) {
-        t_scr[(int64_t)cnt * n_alive + i] = t0;
-        cnt++;
+    if (group && group_usable(g, r)) {
+      alive = G == 16 ? march_group<16>(g, cz, r, n_steps, ts, cnt, bins)
+                      : march_group<4>(g, cz, r, n_steps, ts, cnt, bins);
+    } else {
+      while (cnt < n_steps) {
+        float t0;
+        const int res = march_trip(g, cz, r, t0, bins);
+        if (res == TRIP_END) { alive = false; break; }
+        if (res == TRIP_SAMPLE) {
+          if (group) ts[cnt] = t0;
+          else t_scr[(int64_t)cnt * n_alive + i] = t0;
+          cnt++;
+        }
       }
     }
     rs.t = r.t1;
     rs.j = r.j;
   }
+  // the group's first lane reserves for the ray
   int slot[2];
-  block_reserve<2>({cnt, bins}, {s_counter, step_counter}, slot);
-  const int off = slot[0];
+  block_reserve<2>({sub == 0 ? cnt : 0, sub == 0 ? bins : 0}, {s_counter, step_counter}, slot);
+  const int off = group ? __shfl(slot[0], 0, G) : slot[0];
   if (valid) {
     const V3 o = {rs.ox, rs.oy, rs.oz}, d = {rs.dx, rs.dy, rs.dz};
     const float pxf = __builtin_bit_cast(float, px);
-    // the t0 of EMIT samples are loaded together before they are used
-    for (int k0 = 0; k0 < cnt; k0 += EMIT) {
-      float t0v[EMIT];
+    auto emit = [&](int k, float t0) {
+      const float t1 = t0 + step_dt(mg.st, t0);
+      const float tm = (t0 + t1) * 0.5f;
+      const V3 p = contract(o + tm * d, con);
+      const int64_t q = (int64_t)off + k;
+      s_pos[q] = make_float4(p.x, p.y, p.z, pxf);
+      s_t0[q] = t0;
+    };
+    if (group) {
+      for (int k = sub; k < cnt; k += G) emit(k, ts[k]);
+    } else {
+      // the t0 of EMIT samples are loaded together before they are used
+      for (int k0 = 0; k0 < cnt; k0 += EMIT) {
+        float t0v[EMIT];
 #pragma unroll
-      for (int u = 0; u < EMIT; u++) t0v[u] = t_scr[(int64_t)min(k0 + u, cnt - 1) * n_alive + i];
+        for (int u = 0; u < EMIT; u++) t0v[u] = t_scr[(int64_t)min(k0 + u, cnt - 1) * n_alive + i];
 #pragma unroll
-      for (int u = 0; u < EMIT; u++) {
-        const int k = k0 + u;
-        if (k >= cnt) break;
-        const float t0 = t0v[u];
-        const float t1 = t0 + step_dt(mg.st, t0);
-        const float tm = (t0 + t1) * 0.5f;
-        const V3 p = contract(o + tm * d, con);
-        const int64_t q = (int64_t)off + k;
-        s_pos[q] = make_float4(p.x, p.y, p.z, pxf);
-        s_t0[q] = t0;
+        for (int u = 0; u < EMIT; u++) {
+          if (k0 + u >= cnt) break;
+          emit(k0 + u, t0v[u]);
+        }
       }
     }
-    rays[i] = RayDyn{rs.t, rs.j};
-    entry[i] = make_int4(off, cnt, 0, 0);
-    alive_flag[i] = alive;
+    if (sub == 0) {
+      rays[i] = RayDyn{rs.t, rs.j};
+      entry[i] = make_int4(off, cnt, 0, 0);
+      alive_flag[i] = alive;
+    }
   }
 }
 
@@ -160,9 +180,13 @@ __global__ __launch_bounds__(256) void k_composite(int* __restrict__ ctl, int pa
                                                    RayDyn* __restrict__ rays_out, int* __restrict__ pix_out,
                                                    float4* __restrict__ res_out, float4* __restrict__ results) {
   const int n_alive = ctl[CTL_ALIVE + par];
-  if ((int)(blockIdx.x * blockDim.x) >= n_alive) return;
+  const int G = group_lanes(n_alive);
+  const bool group = G > 1;
+  const int rays_per_block = 256 / G;
+  if ((int)blockIdx.x * rays_per_block >= n_alive) return;
   int* counter = ctl + CTL_ALIVE + (par ^ 1);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
+  const int sub = threadIdx.x & (G - 1);
   const bool valid = i < n_alive;
   bool keep = false;
   int px = 0;
@@ -174,22 +198,33 @@ __global__ __launch_bounds__(256) void k_composite(int* __restrict__ ctl, int pa
     const int ray_alive = alive_flag[i];
     px = pix_in[i];
     bool visible = true;  // transmittance still above the early-stop threshold
-    for (int k0 = 0; k0 < e.y && visible; k0 += COMPOSITE_BATCH) {
-      uint2 v[COMPOSITE_BATCH];
-      float t[COMPOSITE_BATCH];
-#pragma unroll
-      for (int u = 0; u < COMPOSITE_BATCH; u++) {
-        if (k0 + u < e.y) {
-          v[u] = s_out[e.x + k0 + u];
-          t[u] = s_t0[e.x + k0 + u];
-        }
+    if (group) {
+      int n_done = 0;
+      for (int k0 = 0; k0 < e.y && visible; k0 += G) {
+        const int q = e.x + min(k0 + sub, e.y - 1);
+        const uint2 v = s_out[q];
+        const float t = s_t0[q];
+        visible = G == 16 ? composite_group<16>(res, v, t, e.y - k0, st, alpha_thre, n_done)
+                          : composite_group<4>(res, v, t, e.y - k0, st, alpha_thre, n_done);
       }
+    } else {
+      for (int k0 = 0; k0 < e.y && visible; k0 += COMPOSITE_BATCH) {
+        uint2 v[COMPOSITE_BATCH];
+        float t[COMPOSITE_BATCH];
 #pragma unroll
-      for (int u = 0; u < COMPOSITE_BATCH; u++)
-        if (visible && k0 + u < e.y) visible = composite_sample(res, v[u], t[u], st, alpha_thre);
+        for (int u = 0; u < COMPOSITE_BATCH; u++) {
+          if (k0 + u < e.y) {
+            v[u] = s_out[e.x + k0 + u];
+            t[u] = s_t0[e.x + k0 + u];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < COMPOSITE_BATCH; u++)
+          if (visible && k0 + u < e.y) visible = composite_sample(res, v[u], t[u], st, alpha_thre);
+      }
     }
-    keep = visible && ray_alive != 0;
-    if (!keep) results[px] = res;
+    keep = visible && ray_alive != 0 && sub == 0;
+    if (!keep && sub == 0) results[px] = res;
   }
   int slot[1];
   block_reserve<1>({keep ? 1 : 0}, {counter}, slot);
@@ -539,7 +574,7 @@ void render_full(Renderer& r, const Views& vs, fvc_render_stats* stats) {
   const int64_t cap = r.sample_capacity - 64;
   const int64_t target = std::min<int64_t>(vs.target(r.target_batch), cap);
   const int64_t n_bound = std::min<int64_t>(cap, (int64_t)n0 * r.max_steps);  // samples per launch
-  const dim3 grid((n0 + 255) / 256);
+  const dim3 grid(ray_blocks(n0));
   struct Handles { int march, net, comp; };
   std::vector<Handles> hs;
   auto iteration = [&](int it) {
@@ -547,7 +582,7 @@ void render_full(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, target, r.max_steps, cap, 0);
       Handles h;
       ev = P.begin(s);
-      hipLaunchKernelGGL(multi ? k_march<true> : k_march<false>, grid, dim3(256), 0, s, ctl, cur, mg, m.con,
+      hipLaunchKernelGGL(multi ? k_march<true> : k_march<false>, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl, cur, mg, m.con,
                          m.coarse.as<uint32_t>(), r.scene_refs.as<SceneRef>(), r.rays[cur].as<RayDyn>(), r.ray_const.as<RayState>(), r.ray_pix[cur].as<int>(),
                          r.ray_entry.as<int4>(), r.ray_alive.as<int>(), r.t_scratch.as<float>(),
                          r.s_pos.as<float4>(), r.ray_sh.as<uint4>(), r.s_t0.as<float>());
@@ -711,11 +746,11 @@ void render_full_noalloc(Renderer& r, const fvc_raymarch_info& rm, uint8_t* rgba
   FVC_HIP(hipGetLastError());
   const int64_t cap = S - 64;
   const int64_t n_bound = std::min<int64_t>(cap, P * NOALLOC_STEPS);
-  const dim3 grid((unsigned)((P + 255) / 256));
+  const dim3 grid(ray_blocks(P));
   auto iteration = [&](int it) {
     const int cur = it & 1;
     hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, cap, NOALLOC_STEPS, cap, 0);
-    hipLaunchKernelGGL(k_march<false>, grid, dim3(256), 0, s, ctl, cur, mg, m.con, m.coarse.as<uint32_t>(), nullptr,
+    hipLaunchKernelGGL(k_march<false>, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl, cur, mg, m.con, m.coarse.as<uint32_t>(), nullptr,
                        rays[cur], rconst,
                        pix[cur], entry, alive, t_scr, s_pos, ray_sh, s_t0);
     FVC_HIP(hipGetLastError());

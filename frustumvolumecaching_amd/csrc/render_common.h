@@ -125,26 +125,117 @@ __device__ __forceinline__ int classify_sample(const CacheView& cv, V3 oc, V3 dc
 
 __device__ __forceinline__ float h2f(uint32_t bits16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16); }
 
+// Lanes per ray of the marchers and composites for n alive rays.  Where few
+// rays are alive a lane per ray leaves most of the chip idle and the kernel
+// is as long as one ray's chain of loads (row entries, bitfield word, jump),
+// one chain per sample; a group spends one chain per G bins.  With many rays
+// the lanes that test bins of an empty box are work done for nothing, so the
+// group shrinks as the rays grow.  Measured on whole frames (us), G in the
+// order 1 / 4 / 8 / 16 over the whole frame: 256x256 of the small scene 4040
+// / 2570 / 2320 / 2170, reprojected 320x180 1285 / 815 / 715 / 730, 640x360
+// 1725 / 1350 / 1410 / 1690, 1279x717 (its later launches) 3580 / 3270 / 3480 / 3490.
+static const int GROUP16_RAYS = 1 << 15, GROUP4_RAYS = 1 << 19;
+FVC_HD int group_lanes(int n_alive) { return n_alive <= GROUP16_RAYS ? 16 : (n_alive <= GROUP4_RAYS ? 4 : 1); }
+// blocks of 256 threads that take any count of alive rays up to n
+inline unsigned ray_blocks(int64_t n) {
+  int64_t t = n;
+  for (int64_t k : {std::min<int64_t>(n, GROUP16_RAYS), std::min<int64_t>(n, GROUP4_RAYS)})
+    t = std::max(t, k * group_lanes((int)k));
+  return (unsigned)((t + 255) / 256);
+}
+// LDS of a marcher block: the coarse tables of nlvl cascades, then the t0 of
+// the samples of a block's rays (groups)
+inline size_t march_lds(int nlvl) {
+  return (size_t)nlvl * COARSE_WORDS * 4 + (size_t)(256 / 4) * MAX_STEPS_PER_LAUNCH * 4;
+}
+
+// march_trip's loop by a group of G lanes: up to n_steps samples of the ray,
+// their t0 at t0s[0..cnt) (in LDS; the caller orders the reads).  Returns
+// false when the ray ended.  Lanes of a group stay together; groups of a wave
+// need not.
+template <int G>
+__device__ __forceinline__ bool march_group(const MarchGrid& g, const uint32_t* coarse, MarchRay& r, int n_steps,
+                                            float* t0s, int& cnt, int& bins) {
+  const int lane = lane_id(), sub = lane & (G - 1), sh = lane & ~(G - 1);
+  const uint32_t all = (1u << G) - 1u;
+  bool alive = true;
+  while (cnt < n_steps) {
+    float t0, hi;
+    const int res = march_probe(g, coarse, r, r.j + sub, t0, hi);
+    const uint32_t occ = (uint32_t)(__ballot(res == PROBE_SAMPLE) >> sh) & all;
+    const uint32_t past = (uint32_t)(__ballot(res == PROBE_PAST) >> sh) & all;
+    const GroupPlan p = group_plan(G, occ, past, n_steps - cnt);
+    if ((p.samples >> sub) & 1u) t0s[cnt + __popc(p.samples & ((1u << sub) - 1u))] = t0;
+    cnt += __popc(p.samples);
+    bins += p.bins;
+    r.j += p.bins;
+    if (p.ended) {
+      alive = false;
+      bins++;
+      break;
+    }
+    if (p.full) break;
+#pragma unroll
+    for (int d = 1; d < G; d <<= 1) hi = fmaxf(hi, __shfl_xor(hi, d, G));
+    if (hi > 0.0f) bins += table_jump(g.tab, r.row, r.m, r.j, r.t1, hi);
+  }
+  r.t1 = g.tab.t[r.row.base + r.j];
+  return alive;
+}
+
 // One step of front-to-back compositing (accumulate_performance_kernel,
 // performance_renderer.cu:93-120): v = half4 (r, g, b raw, log sigma).
-// Returns false once T < 1e-4.
-__device__ __forceinline__ bool composite_sample(float4& res, uint2 v, float t0, const fvc_stepsize_info& st,
-                                                 float alpha_thre) {
-  const float cr = h2f(v.x & 0xffffu), cg = h2f(v.x >> 16), cb = h2f(v.y & 0xffffu), ls = h2f(v.y >> 16);
+// composite_alpha: the sample's opacity; composite_add: its colour and the
+// transmittance after it; false once T < 1e-4.
+__device__ __forceinline__ float composite_alpha(uint2 v, float t0, const fvc_stepsize_info& st) {
+  const float ls = h2f(v.y >> 16);
   const float density = expf(ls);
   const float dt = step_dt(st, t0);
-  float alpha = 1.0f - expf(-density * dt);
-  alpha = fminf_(fmaxf_(alpha, 0.0f), 1.0f);
+  const float alpha = 1.0f - expf(-density * dt);
+  return fminf_(fmaxf_(alpha, 0.0f), 1.0f);
+}
+__device__ __forceinline__ V3 composite_colour(uint2 v) {
+  const float cr = h2f(v.x & 0xffffu), cg = h2f(v.x >> 16), cb = h2f(v.y & 0xffffu);
+  return V3{1.0f / (1.0f + expf(-cr)), 1.0f / (1.0f + expf(-cg)), 1.0f / (1.0f + expf(-cb))};
+}
+__device__ __forceinline__ bool composite_add(float4& res, float alpha, V3 c, float alpha_thre) {
   if (alpha > alpha_thre) {
     const float w = alpha * res.w;
-    res.x = res.x + w * (1.0f / (1.0f + expf(-cr)));
-    res.y = res.y + w * (1.0f / (1.0f + expf(-cg)));
-    res.z = res.z + w * (1.0f / (1.0f + expf(-cb)));
+    res.x = res.x + w * c.x;
+    res.y = res.y + w * c.y;
+    res.z = res.z + w * c.z;
     res.w = res.w * (1.0f - alpha);
   }
   return !(res.w < 1e-4f);
 }
-
+__device__ __forceinline__ bool composite_sample(float4& res, uint2 v, float t0, const fvc_stepsize_info& st,
+                                                 float alpha_thre) {
+  const float alpha = composite_alpha(v, t0, st);
+  if (!(alpha > alpha_thre)) return !(res.w < 1e-4f);
+  return composite_add(res, alpha, composite_colour(v), alpha_thre);
+}
+// Up to G samples by a lane group, lane k holding sample k (n of them):
+// opacities and colours in parallel, then every lane runs the sequential
+// products of composite_add in order, so res is the same on all of them and
+// the same as one lane's.  Returns whether the ray stays visible; n_done
+// counts the samples composited.
+template <int G>
+__device__ __forceinline__ bool composite_group(float4& res, uint2 v, float t0, int n, const fvc_stepsize_info& st,
+                                                float alpha_thre, int& n_done) {
+  const float alpha = composite_alpha(v, t0, st);
+  const V3 c = composite_colour(v);
+  bool visible = true;
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    const float au = __shfl(alpha, u, G);
+    const V3 cu = V3{__shfl(c.x, u, G), __shfl(c.y, u, G), __shfl(c.z, u, G)};
+    if (u < n && visible) {
+      visible = composite_add(res, au, cu, alpha_thre);
+      n_done++;
+    }
+  }
+  return visible;
+}
 // to_8bit (raymarch_common.h:554-557)
 FVC_HD int to_8bit(float f) {
   const int v = (int)(f * 256.0f);
