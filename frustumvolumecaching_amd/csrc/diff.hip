@@ -286,32 +286,61 @@ __device__ __forceinline__ void net_forward(const float4* fr, const float* __res
 __device__ __forceinline__ V3 ray_dir01(const RayState& r) { return unit_to_01(V3{r.dx, r.dy, r.dz}); }
 
 // ------------------------------------------------------------ march
+// Every ray is marched to its far bound, by G lanes each (group_lanes; a
+// batch of a few thousand rays would otherwise wait for its longest ray).
+// each(is, t0): is: the lane holds a sample, of start t0; called by all lanes
+// of a group together, in march order.
+template <int G, class Each>
+__device__ __forceinline__ void march_all(const MarchGrid& mg, const uint32_t* coarse, MarchRay& mr, Each&& each) {
+  int bins = 0, cnt = 0;
+  const int sub = lane_id() & (G - 1);
+  if (G > 1 && group_usable(mg, mr)) {
+    march_group_steps<(G > 1 ? G : 2)>(mg, coarse, mr, 0x7fffffff, cnt, bins, [&](uint32_t samples, int, float t0) {
+      each(((samples >> sub) & 1u) != 0u, t0);
+    });
+    return;
+  }
+  while (true) {
+    float t0;
+    const int res = march_trip(mg, coarse, mr, t0, bins);
+    if (res == TRIP_END) break;
+    if (res == TRIP_SAMPLE) each(sub == 0, t0);
+  }
+}
+// lanes of the group with is set below this one, and in all
+template <int G> __device__ __forceinline__ int group_rank(bool is, int& total) {
+  const int lane = lane_id(), sub = lane & (G - 1), sh = lane & ~(G - 1);
+  const uint32_t m = (uint32_t)(__ballot(is) >> sh) & ((1u << G) - 1u);
+  total = __popc(m);
+  return __popc(m & ((1u << sub) - 1u));
+}
+
+template <int G>
 __global__ __launch_bounds__(256) void k_diff_count(fvc_raymarch_info rm, V3 aabb_from, V3 aabb_to,
                                                     const int* __restrict__ pix, int n, MarchGrid mg,
                                                     const uint32_t* __restrict__ coarse_g,
                                                     RayState* __restrict__ rays, int* __restrict__ counts) {
   __shared__ uint32_t coarse[16 * COARSE_WORDS];
   load_coarse(coarse_g, mg.occ.nlvl, coarse);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * (256 / G) + threadIdx.x / G, sub = threadIdx.x & (G - 1);
   if (i >= n) return;
   const int W = rm.cam_info.res_x;
   RayState r;
   const bool hit = init_ray_state(rm, aabb_from, aabb_to, pix[i] % W, pix[i] / W, r);
-  rays[i] = r;
+  if (sub == 0) rays[i] = r;
   int cnt = 0;
   if (hit) {
     MarchRay mr = march_ray(r, mg.tab);
-    int bins = 0;
-    while (true) {
-      float t0;
-      const int res = march_trip(mg, coarse, mr, t0, bins);
-      if (res == TRIP_END) break;
-      if (res == TRIP_SAMPLE) cnt++;
-    }
+    march_all<G>(mg, coarse, mr, [&](bool is, float) {
+      int total;
+      group_rank<G>(is, total);
+      cnt += total;
+    });
   }
-  counts[i] = cnt;
+  if (sub == 0) counts[i] = cnt;
 }
 
+template <int G>
 __global__ __launch_bounds__(256) void k_diff_emit(int n, MarchGrid mg, ContractParams con,
                                                    const uint32_t* __restrict__ coarse_g,
                                                    const RayState* __restrict__ rays, const int* __restrict__ counts,
@@ -319,27 +348,24 @@ __global__ __launch_bounds__(256) void k_diff_emit(int n, MarchGrid mg, Contract
                                                    float* __restrict__ s_dt, int* __restrict__ s_ray) {
   __shared__ uint32_t coarse[16 * COARSE_WORDS];
   load_coarse(coarse_g, mg.occ.nlvl, coarse);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * (256 / G) + threadIdx.x / G;
   if (i >= n || counts[i] == 0) return;
   const RayState r = rays[i];
   MarchRay mr = march_ray(r, mg.tab);
   const V3 o = {r.ox, r.oy, r.oz}, d = {r.dx, r.dy, r.dz};
-  int q = (int)offsets[i];  // the batch holds fewer than 2^31 samples
-  const int end = q + counts[i];
-  int bins = 0;
-  while (q < end) {
-    float t0;
-    const int res = march_trip(mg, coarse, mr, t0, bins);
-    if (res == TRIP_END) break;
-    if (res != TRIP_SAMPLE) continue;
+  int q0 = (int)offsets[i];  // the batch holds fewer than 2^31 samples
+  march_all<G>(mg, coarse, mr, [&](bool is, float t0) {
+    int total;
+    const int q = q0 + group_rank<G>(is, total);
+    q0 += total;
+    if (!is) return;
     const float dt = step_dt(mg.st, t0);
     const float tm = (t0 + (t0 + dt)) * 0.5f;
     const V3 p = contract(o + tm * d, con);
-    s_pos[3 * q] = p.x; s_pos[3 * q + 1] = p.y; s_pos[3 * q + 2] = p.z;
+    s_pos[3 * (int64_t)q] = p.x; s_pos[3 * (int64_t)q + 1] = p.y; s_pos[3 * (int64_t)q + 2] = p.z;
     s_dt[q] = dt;
     s_ray[q] = i;
-    q++;
-  }
+  });
 }
 
 // ------------------------------------------------------------ network
@@ -378,32 +404,47 @@ __device__ __forceinline__ void sample_terms(float4 o4, float dt, float& sigma, 
   c[2] = 1.0f / (1.0f + expf(-o4.z));
 }
 
+// Both composites: G lanes per ray, lane k taking sample k of the next G; the
+// terms of a sample are formed on its lane, the sequential products in march
+// order on every lane, so the results do not depend on G.
+template <int G>
 __global__ __launch_bounds__(256) void k_diff_composite(int n, float alpha_thre, const int* __restrict__ counts,
                                                         const int64_t* __restrict__ offsets,
                                                         const float4* __restrict__ out4,
                                                         const float* __restrict__ s_dt, float* __restrict__ rgb,
                                                         float4* __restrict__ ray_out, int* __restrict__ n_used) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * (256 / G) + threadIdx.x / G, sub = threadIdx.x & (G - 1);
   if (i >= n) return;
   const int off = (int)offsets[i], cnt = counts[i];
   float C[3] = {0.0f, 0.0f, 0.0f}, T = 1.0f;
-  int k = 0;
-  for (; k < cnt; k++) {
+  int k = 0;  // samples walked
+  bool ended = false;
+  for (int k0 = 0; k0 < cnt && !ended; k0 += G) {
     float sigma, alpha, c[3];
-    sample_terms(out4[off + k], s_dt[off + k], sigma, alpha, c);
-    if (alpha > alpha_thre) {
-      const float w = alpha * T;
-      for (int ch = 0; ch < 3; ch++) C[ch] = C[ch] + w * c[ch];
-      T = T * (1.0f - alpha);
+    const int q = off + min(k0 + sub, cnt - 1);
+    sample_terms(out4[q], s_dt[q], sigma, alpha, c);
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const float au = __shfl(alpha, u, G);
+      const float cu[3] = {__shfl(c[0], u, G), __shfl(c[1], u, G), __shfl(c[2], u, G)};
+      if (k0 + u >= cnt || ended) continue;
+      if (au > alpha_thre) {
+        const float w = au * T;
+        for (int ch = 0; ch < 3; ch++) C[ch] = C[ch] + w * cu[ch];
+        T = T * (1.0f - au);
+      }
+      k++;
+      ended = T < 1e-4f;
     }
-    if (T < 1e-4f) { k++; break; }
   }
+  if (sub != 0) return;
   const float4 res = make_float4(C[0] + T, C[1] + T, C[2] + T, T);
   ray_out[i] = res;
-  n_used[i] = k;  // samples walked (the backward walks the same ones)
+  n_used[i] = k;  // the backward walks the same ones
   rgb[3 * i] = res.x; rgb[3 * i + 1] = res.y; rgb[3 * i + 2] = res.z;
 }
 
+template <int G>
 __global__ __launch_bounds__(256) void k_diff_composite_bwd(int n, float alpha_thre, const int* __restrict__ counts,
                                                             const int64_t* __restrict__ offsets,
                                                             const int* __restrict__ n_walk,
@@ -412,34 +453,48 @@ __global__ __launch_bounds__(256) void k_diff_composite_bwd(int n, float alpha_t
                                                             const float4* __restrict__ ray_out,
                                                             const float* __restrict__ d_rgb,
                                                             float4* __restrict__ d_out4) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * (256 / G) + threadIdx.x / G, sub = threadIdx.x & (G - 1);
   if (i >= n) return;
   const int off = (int)offsets[i], cnt = counts[i], walk = n_walk[i];
   const float4 ro = ray_out[i];
   const float tot[3] = {ro.x, ro.y, ro.z};
   const float dr[3] = {d_rgb[3 * i], d_rgb[3 * i + 1], d_rgb[3 * i + 2]};
   float T = 1.0f, pre[3] = {0.0f, 0.0f, 0.0f};
-  for (int k = 0; k < cnt; k++) {
+  for (int k0 = 0; k0 < cnt; k0 += G) {
+    const int k = k0 + sub;
     float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (k < walk) {
-      const float dt = s_dt[off + k];
+    if (k0 < walk) {
       float sigma, alpha, c[3];
-      sample_terms(out4[off + k], dt, sigma, alpha, c);
-      if (alpha > alpha_thre) {
-        const float w = alpha * T;
-        const float T1 = T * (1.0f - alpha);
+      const int q = off + min(k, walk - 1);
+      const float dt = s_dt[q];
+      sample_terms(out4[q], dt, sigma, alpha, c);
+      // the lane's own sample: weight, transmittance after it, colour up to it
+      float wk = 0.0f, T1 = 0.0f, pk[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const float au = __shfl(alpha, u, G);
+        const float cu[3] = {__shfl(c[0], u, G), __shfl(c[1], u, G), __shfl(c[2], u, G)};
+        if (k0 + u >= walk || !(au > alpha_thre)) continue;
+        const float w = au * T;
+        T = T * (1.0f - au);
+        for (int ch = 0; ch < 3; ch++) pre[ch] = pre[ch] + w * cu[ch];
+        if (u == sub) {
+          wk = w;
+          T1 = T;
+          for (int ch = 0; ch < 3; ch++) pk[ch] = pre[ch];
+        }
+      }
+      if (k < walk && alpha > alpha_thre) {
         float dsig = 0.0f, dc[3];
         for (int ch = 0; ch < 3; ch++) {
-          pre[ch] = pre[ch] + w * c[ch];
-          const float S = tot[ch] - pre[ch];
+          const float S = tot[ch] - pk[ch];
           dsig = dsig + dr[ch] * (T1 * c[ch] - S);
-          dc[ch] = dr[ch] * w * c[ch] * (1.0f - c[ch]);
+          dc[ch] = dr[ch] * wk * c[ch] * (1.0f - c[ch]);
         }
         d = make_float4(dc[0], dc[1], dc[2], dsig * dt * sigma);
-        T = T1;
       }
     }
-    d_out4[off + k] = d;
+    if (k < cnt) d_out4[off + k] = d;
   }
 }
 
@@ -951,6 +1006,7 @@ __global__ __launch_bounds__(64 * BWD_WAVES) void k_diff_net_bwd(int j0, int n, 
 //   dL/dl_c,i   = w_c dL/dl_i / sum_c w_c isset_c;
 // isset is a mask.  Voxel gradients go to g_pool [slot][512][10] (8 latents,
 // density, isset = 0) with FP32 atomics.
+template <int G>
 __global__ __launch_bounds__(256) void k_diffc_count(fvc_raymarch_info rm, V3 aabb_from, V3 aabb_to,
                                                      const int* __restrict__ pix, int n, MarchGrid mg, CacheView cv,
                                                      const uint32_t* __restrict__ coarse_g,
@@ -958,32 +1014,33 @@ __global__ __launch_bounds__(256) void k_diffc_count(fvc_raymarch_info rm, V3 aa
                                                      int* __restrict__ counts_c) {
   __shared__ uint32_t coarse[16 * COARSE_WORDS];
   load_coarse(coarse_g, mg.occ.nlvl, coarse);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * (256 / G) + threadIdx.x / G, sub = threadIdx.x & (G - 1);
   if (i >= n) return;
   const int W = rm.cam_info.res_x;
   RayState r;
   const bool hit = init_ray_state(rm, aabb_from, aabb_to, pix[i] % W, pix[i] / W, r);
-  rays[i] = r;
+  if (sub == 0) rays[i] = r;
   int nr = 0, nc = 0;
   if (hit) {
     MarchRay mr = march_ray(r, mg.tab);
     const V3 oc = transform(cv.cam.world2cam, mr.o.x, mr.o.y, mr.o.z, 1.0f);
     const V3 dc = transform(cv.cam.world2cam, mr.d.x, mr.d.y, mr.d.z, 0.0f);
-    int bins = 0;
-    while (true) {
-      float t0;
-      const int res = march_trip(mg, coarse, mr, t0, bins);
-      if (res == TRIP_END) break;
-      if (res != TRIP_SAMPLE) continue;
-      const int k = classify_sample(cv, oc, dc, t0, step_dt(mg.st, t0));
-      nr += k == SAMPLE_RESAMPLE;
-      nc += k == SAMPLE_CACHE;
-    }
+    march_all<G>(mg, coarse, mr, [&](bool is, float t0) {
+      const int k = is ? classify_sample(cv, oc, dc, t0, step_dt(mg.st, t0)) : SAMPLE_SKIP;
+      int tr, tc;
+      group_rank<G>(k == SAMPLE_RESAMPLE, tr);
+      group_rank<G>(k == SAMPLE_CACHE, tc);
+      nr += tr;
+      nc += tc;
+    });
   }
-  counts_r[i] = nr;
-  counts_c[i] = nc;
+  if (sub == 0) {
+    counts_r[i] = nr;
+    counts_c[i] = nc;
+  }
 }
 
+template <int G>
 __global__ __launch_bounds__(256) void k_diffc_emit(int n, MarchGrid mg, ContractParams con, CacheView cv,
                                                     const uint32_t* __restrict__ coarse_g,
                                                     const RayState* __restrict__ rays,
@@ -995,45 +1052,46 @@ __global__ __launch_bounds__(256) void k_diffc_emit(int n, MarchGrid mg, Contrac
                                                     int* __restrict__ list_r, int* __restrict__ list_c) {
   __shared__ uint32_t coarse[16 * COARSE_WORDS];
   load_coarse(coarse_g, mg.occ.nlvl, coarse);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * (256 / G) + threadIdx.x / G, sub = threadIdx.x & (G - 1);
   if (i >= n) return;
   const int nr = counts_r[i], nc = counts_c[i];
-  int q = (int)(off_r[i] + off_c[i]);  // the batch holds fewer than 2^31 samples
-  counts[i] = nr + nc;
-  offsets[i] = q;
+  int q0 = (int)(off_r[i] + off_c[i]);  // the batch holds fewer than 2^31 samples
+  if (sub == 0) {
+    counts[i] = nr + nc;
+    offsets[i] = q0;
+  }
   if (nr + nc == 0) return;
   const RayState r = rays[i];
   MarchRay mr = march_ray(r, mg.tab);
   const V3 o = {r.ox, r.oy, r.oz}, d = {r.dx, r.dy, r.dz};
   const V3 oc = transform(cv.cam.world2cam, o.x, o.y, o.z, 1.0f);
   const V3 dc = transform(cv.cam.world2cam, d.x, d.y, d.z, 0.0f);
-  int kr = (int)off_r[i], kc = (int)off_c[i];
-  const int end = q + nr + nc;
-  int bins = 0;
-  while (q < end) {
-    float t0;
-    const int res = march_trip(mg, coarse, mr, t0, bins);
-    if (res == TRIP_END) break;
-    if (res != TRIP_SAMPLE) continue;
+  int kr0 = (int)off_r[i], kc0 = (int)off_c[i];
+  march_all<G>(mg, coarse, mr, [&](bool is, float t0) {
     const float dt = step_dt(mg.st, t0);
-    const int k = classify_sample(cv, oc, dc, t0, dt);
-    if (k == SAMPLE_SKIP) continue;
+    const int k = is ? classify_sample(cv, oc, dc, t0, dt) : SAMPLE_SKIP;
+    int tr, tc;
+    const int kr = kr0 + group_rank<G>(k == SAMPLE_RESAMPLE, tr), kc = kc0 + group_rank<G>(k == SAMPLE_CACHE, tc);
+    const int q = q0 + (kr - kr0) + (kc - kc0);
+    kr0 += tr;
+    kc0 += tc;
+    q0 += tr + tc;
+    if (k == SAMPLE_SKIP) return;
     // network inputs at t0 + dt / 2 (cache_performance_renderer.cu:198-313)
     const float tm2 = t0 + dt * 0.5f;
     V3 p;
     if (k == SAMPLE_RESAMPLE) {
       p = contract(o + tm2 * d, con);
-      list_r[kr++] = q;
+      list_r[kr] = q;
     } else {
       float tf;
       p = cam2froxel(oc + tm2 * dc, cv.cam, cv.st, tf);
-      list_c[kc++] = q;
+      list_c[kc] = q;
     }
-    s_pos[3 * q] = p.x; s_pos[3 * q + 1] = p.y; s_pos[3 * q + 2] = p.z;
+    s_pos[3 * (int64_t)q] = p.x; s_pos[3 * (int64_t)q + 1] = p.y; s_pos[3 * (int64_t)q + 2] = p.z;
     s_dt[q] = dt;
     s_ray[q] = i;
-    q++;
-  }
+  });
 }
 
 // trilinear lookup of one sample by its 4 lanes: lane group g fetches the
@@ -1223,6 +1281,9 @@ static int persistent_blocks(int64_t n_groups) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(blocks, 256 * 8));
 }
 
+// the kernel of G lanes per ray
+#define BY_LANES(G, k) ((G) == 16 ? k<16> : ((G) == 4 ? k<4> : k<1>))
+
 // blocks of the backward kernels: one per CU (their fragments and staging
 // rows fill its LDS), 128 samples per block and iteration
 static int bwd_blocks(int64_t n) {
@@ -1328,10 +1389,11 @@ void diff_forward(Renderer& r, const fvc_raymarch_info& rm, const int* pix, int 
   const MarchGrid mg = march_grid(r, &rm, 1);
   const V3 af = {m.scene.aabb_from.x, m.scene.aabb_from.y, m.scene.aabb_from.z};
   const V3 at = {m.scene.aabb_to.x, m.scene.aabb_to.y, m.scene.aabb_to.z};
-  const dim3 grid((n + 255) / 256);
+  const int G = mg.tab.n_rows > 0 ? group_lanes(n) : 1;
+  const dim3 grid((unsigned)(((int64_t)n * G + 255) / 256));
   int64_t total64 = 0;
   if (!cached) {
-    hipLaunchKernelGGL(k_diff_count, grid, dim3(256), 0, s, rm, af, at, pix, n, mg, m.coarse.as<uint32_t>(),
+    hipLaunchKernelGGL(BY_LANES(G, k_diff_count), grid, dim3(256), 0, s, rm, af, at, pix, n, mg, m.coarse.as<uint32_t>(),
                        D.rays.as<RayState>(), D.counts.as<int>());
     FVC_HIP(hipGetLastError());
     total64 = scan_counts(D, D.counts.as<int>(), D.offsets.as<int64_t>(), n, s);
@@ -1341,7 +1403,7 @@ void diff_forward(Renderer& r, const fvc_raymarch_info& rm, const int* pix, int 
     D.counts_c.ensure(((size_t)n + 1) * sizeof(int));
     D.off_r.ensure(((size_t)n + 1) * sizeof(int64_t));
     D.off_c.ensure(((size_t)n + 1) * sizeof(int64_t));
-    hipLaunchKernelGGL(k_diffc_count, grid, dim3(256), 0, s, rm, af, at, pix, n, mg, D.cv, m.coarse.as<uint32_t>(),
+    hipLaunchKernelGGL(BY_LANES(G, k_diffc_count), grid, dim3(256), 0, s, rm, af, at, pix, n, mg, D.cv, m.coarse.as<uint32_t>(),
                        D.rays.as<RayState>(), D.counts.as<int>(), D.counts_c.as<int>());
     FVC_HIP(hipGetLastError());
     D.n_r = scan_counts(D, D.counts.as<int>(), D.off_r.as<int64_t>(), n, s);
@@ -1359,14 +1421,14 @@ void diff_forward(Renderer& r, const fvc_raymarch_info& rm, const int* pix, int 
   D.out4.ensure(ns * sizeof(float4));
   D.d_out4.ensure(ns * sizeof(float4));
   if (!cached) {
-    hipLaunchKernelGGL(k_diff_emit, grid, dim3(256), 0, s, n, mg, m.con, m.coarse.as<uint32_t>(),
+    hipLaunchKernelGGL(BY_LANES(G, k_diff_emit), grid, dim3(256), 0, s, n, mg, m.con, m.coarse.as<uint32_t>(),
                        D.rays.as<RayState>(), D.counts.as<int>(), D.offsets.as<int64_t>(), D.s_pos.as<float>(),
                        D.s_dt.as<float>(), D.s_ray.as<int>());
   } else {
     D.list_r.ensure((size_t)std::max<int64_t>(D.n_r, 1) * sizeof(int));
     D.list_c.ensure((size_t)std::max<int64_t>(D.n_c, 1) * sizeof(int));
     D.counts_all.ensure((size_t)n * sizeof(int));
-    hipLaunchKernelGGL(k_diffc_emit, grid, dim3(256), 0, s, n, mg, m.con, D.cv, m.coarse.as<uint32_t>(),
+    hipLaunchKernelGGL(BY_LANES(G, k_diffc_emit), grid, dim3(256), 0, s, n, mg, m.con, D.cv, m.coarse.as<uint32_t>(),
                        D.rays.as<RayState>(), D.counts.as<int>(), D.counts_c.as<int>(), D.off_r.as<int64_t>(),
                        D.off_c.as<int64_t>(), D.counts_all.as<int>(), D.offsets.as<int64_t>(), D.s_pos.as<float>(),
                        D.s_dt.as<float>(), D.s_ray.as<int>(), D.list_r.as<int>(), D.list_c.as<int>());
@@ -1386,7 +1448,7 @@ void diff_forward(Renderer& r, const fvc_raymarch_info& rm, const int* pix, int 
     FVC_HIP(hipGetLastError());
   }
   const int* counts = cached ? D.counts_all.as<int>() : D.counts.as<int>();
-  hipLaunchKernelGGL(k_diff_composite, grid, dim3(256), 0, s, n, m.scene.alpha_thre, counts, D.offsets.as<int64_t>(),
+  hipLaunchKernelGGL(BY_LANES(G, k_diff_composite), grid, dim3(256), 0, s, n, m.scene.alpha_thre, counts, D.offsets.as<int64_t>(),
                      D.out4.as<float4>(), D.s_dt.as<float>(), rgb, D.ray_out.as<float4>(), D.n_walk.as<int>());
   FVC_HIP(hipGetLastError());
   FVC_HIP(hipStreamSynchronize(s));
@@ -1409,7 +1471,8 @@ void diff_backward(Renderer& r, const float* d_rgb, float* g_pos, float* g_base,
   const int n = D.n;
   if (n == 0) return;
   const int* counts = D.cached ? D.counts_all.as<int>() : D.counts.as<int>();
-  hipLaunchKernelGGL(k_diff_composite_bwd, dim3((n + 255) / 256), dim3(256), 0, s, n, m.scene.alpha_thre, counts,
+  const int G = group_lanes(n);
+  hipLaunchKernelGGL(BY_LANES(G, k_diff_composite_bwd), dim3((unsigned)(((int64_t)n * G + 255) / 256)), dim3(256), 0, s, n, m.scene.alpha_thre, counts,
                      D.offsets.as<int64_t>(), D.n_walk.as<int>(), D.out4.as<float4>(), D.s_dt.as<float>(),
                      D.ray_out.as<float4>(), d_rgb, D.d_out4.as<float4>());
   FVC_HIP(hipGetLastError());

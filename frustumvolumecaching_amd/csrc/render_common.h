@@ -149,13 +149,14 @@ inline size_t march_lds(int nlvl) {
   return (size_t)nlvl * COARSE_WORDS * 4 + (size_t)(256 / 4) * MAX_STEPS_PER_LAUNCH * 4;
 }
 
-// march_trip's loop by a group of G lanes: up to n_steps samples of the ray,
-// their t0 at t0s[0..cnt) (in LDS; the caller orders the reads).  Returns
-// false when the ray ended.  Lanes of a group stay together; groups of a wave
-// need not.
-template <int G>
-__device__ __forceinline__ bool march_group(const MarchGrid& g, const uint32_t* coarse, MarchRay& r, int n_steps,
-                                            float* t0s, int& cnt, int& bins) {
+// march_trip's loop by a group of G lanes, up to n_steps samples of the ray.
+// Every step calls step(samples, cnt, t0) on all lanes of the group: bit k of
+// samples marks lane k's bin, of start t0 on that lane, as a sample; cnt
+// samples came before.  Returns false when the ray ended.  Lanes of a group
+// stay together; groups of a wave need not.
+template <int G, class Step>
+__device__ __forceinline__ bool march_group_steps(const MarchGrid& g, const uint32_t* coarse, MarchRay& r, int n_steps,
+                                                  int& cnt, int& bins, Step&& step) {
   const int lane = lane_id(), sub = lane & (G - 1), sh = lane & ~(G - 1);
   const uint32_t all = (1u << G) - 1u;
   bool alive = true;
@@ -165,7 +166,7 @@ __device__ __forceinline__ bool march_group(const MarchGrid& g, const uint32_t* 
     const uint32_t occ = (uint32_t)(__ballot(res == PROBE_SAMPLE) >> sh) & all;
     const uint32_t past = (uint32_t)(__ballot(res == PROBE_PAST) >> sh) & all;
     const GroupPlan p = group_plan(G, occ, past, n_steps - cnt);
-    if ((p.samples >> sub) & 1u) t0s[cnt + __popc(p.samples & ((1u << sub) - 1u))] = t0;
+    step(p.samples, cnt, t0);
     cnt += __popc(p.samples);
     bins += p.bins;
     r.j += p.bins;
@@ -181,6 +182,15 @@ __device__ __forceinline__ bool march_group(const MarchGrid& g, const uint32_t* 
   }
   r.t1 = g.tab.t[r.row.base + r.j];
   return alive;
+}
+// ... with the samples' t0 at t0s[0..cnt) (in LDS; the caller orders the reads)
+template <int G>
+__device__ __forceinline__ bool march_group(const MarchGrid& g, const uint32_t* coarse, MarchRay& r, int n_steps,
+                                            float* t0s, int& cnt, int& bins) {
+  const int sub = lane_id() & (G - 1);
+  return march_group_steps<G>(g, coarse, r, n_steps, cnt, bins, [&](uint32_t samples, int before, float t0) {
+    if ((samples >> sub) & 1u) t0s[before + __popc(samples & ((1u << sub) - 1u))] = t0;
+  });
 }
 
 // One step of front-to-back compositing (accumulate_performance_kernel,
