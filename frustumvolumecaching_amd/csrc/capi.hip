@@ -150,8 +150,9 @@ static void create_model(const fvc_scene_info* scene, const fvc_net_desc* net, c
       const std::vector<uint32_t> coarse = build_coarse(occ, scene->grid_nlvl);
       m.coarse.ensure(coarse.size() * sizeof(uint32_t));
       FVC_HIP(hipMemcpy(m.coarse.p, coarse.data(), coarse.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-      m.table.ensure(n_pos * sizeof(uint16_t));
+      m.table.ensure(n_pos * sizeof(uint16_t) + plan_copies(m.grid, n_pos / 2) * sizeof(uint32_t));
       FVC_HIP(hipMemcpy(m.table.p, p_pos, n_pos * sizeof(uint16_t), hipMemcpyHostToDevice));
+      fill_copies(m.grid, m.table.as<uint32_t>());
       std::vector<uint8_t> frags;
       if (net->split_head) pack_fragments_vd(p_base, p_first, p_head, *net, frags);
       else pack_fragments(p_base, p_head, net->precision, net->latent_offset, net->n_latents, frags, m.mlp_scales);

@@ -66,12 +66,22 @@ struct GridLevel {
   uint32_t res2;     // res * res
   uint32_t size;     // entries in the level
   uint32_t offset;   // first entry of the level
-  uint32_t first;    // the value of that entry (set by the kernels' level copy)
+};
+// A level as the FP16 encoder reads it, from Model::table (byte offsets):
+// copied levels at off + 4 x + ya y + za z, hashed ones at off + ((4 x ^ ya y
+// ^ za z) & mask).
+struct EncLevel {
+  float scale;
+  uint32_t ya, za;   // byte strides, or 4 times the hash primes
+  uint32_t off;
+  uint32_t mask;     // hashed: 4 (entries - 1)
 };
 struct GridParams {
   GridLevel lv[MAX_LEVELS];
   uint32_t dense_mask;  // bit l: level l indexed densely
-  uint32_t quad_dense;  // bit j: levels 4j..4j+3 all dense
+  EncLevel enc[MAX_LEVELS];
+  uint32_t copy_mask;   // bit l: the encoder reads a vertex copy of level l (plan_copies)
+  uint32_t quad_copy;   // bit j: levels 4j..4j+3 all copied
   uint32_t quad_hash;   // bit j: levels 4j..4j+3 all hashed
   int n_levels;
 };
@@ -112,7 +122,7 @@ struct Model {
   int64_t n_pos_enc = 0, n_base = 0, n_head = 0, n_first = 0;
   DevBuf bitfield;   // Morton occupancy bitfield
   DevBuf coarse;     // per cascade 16^3 "any of 8^3 cells occupied" bits
-  DevBuf table;      // hash grid, uint32 per entry (2 x fp16)
+  DevBuf table;      // hash grid, uint32 per entry (2 x fp16), then the vertex copies of its coarse levels
   DevBuf frags;      // packed weight fragments in the MLP precision
   MlpScales mlp_scales{};
   std::vector<uint8_t> bitfield_host;
@@ -136,6 +146,11 @@ inline int vd_head_inputs(const fvc_net_desc& d) { return (8 + 16 + 16 + 6 * d.f
 // (split models: mlp_first_head) is 0 for plain models
 bool net_layout(const fvc_net_desc& d, GridParams& g, int64_t& n_pos, int64_t& n_base, int64_t& n_head,
                 int64_t* n_first = nullptr);
+
+// entries of the vertex copies behind a table of n_entries; fills the encoder's view of g
+int64_t plan_copies(GridParams& g, int64_t n_entries);
+// writes the copies planned in g into the table (device)
+void fill_copies(const GridParams& g, uint32_t* table);
 
 // model export of the reference (loader.hip)
 struct NerfaccExport {

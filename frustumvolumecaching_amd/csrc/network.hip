@@ -73,11 +73,6 @@ bool net_layout(const fvc_net_desc& d, GridParams& g, int64_t& n_pos, int64_t& n
     if (dense <= p) g.dense_mask |= 1u << l;
     off += (uint32_t)p;
   }
-  for (int j = 0; j < 4; j++) {
-    const uint32_t q = (g.dense_mask >> (4 * j)) & 15u;
-    if (q == 15u) g.quad_dense |= 1u << j;
-    if (q == 0u) g.quad_hash |= 1u << j;
-  }
   n_pos = (int64_t)off * 2;
   n_base = 32 * 64 + 64 * 64 + 64 * 16;
   n_head = 32 * 64 + 64 * 16;
@@ -90,101 +85,219 @@ bool net_layout(const fvc_net_desc& d, GridParams& g, int64_t& n_pos, int64_t& n
 }
 
 // ------------------------------------------------------------------ encode
-// Entries of corners x and x + 1 of one (y, z) row of a level, with one
-// 8-byte load (dword aligned) for both where the table allows.  ky, kz: the
-// row's y / z index terms (products for dense levels, hash terms otherwise).
-//  * dense: entries a and a + 1 (a = the row's x index reduced to the
-//    level); only when a is the level's last entry does a + 1 wrap to entry
-//    0: then the pair (a - 1, a) is read and corner x + 1 takes L.first.
-//  * hashed (the level's size is a power of two): for even x, x and x + 1
-//    differ in bit 0 only, so their entries i0 and i0 ^ 1 form the aligned
-//    pair holding i0; for odd x corner x + 1 is a load of its own, made by
-//    those lanes only.
-// No branch waits on a load, so every gather of a level is in flight before
-// the first wait.
-__device__ __forceinline__ void row_pair(const uint32_t* __restrict__ tl, const GridLevel& L, bool dense, uint32_t gx,
-                                         uint32_t ky, uint32_t kz, uint32_t& e0, uint32_t& e1) {
-  uint32_t lo, i1 = 0u;
-  bool sel, use_first = false, use_extra = false;
-  if (dense) {
-    const uint32_t t = gx + ky + kz;  // t + 1 < 2 * size
-    const uint32_t a = min(t, t - L.size);
-    const bool pair = a + 1u < L.size;
-    lo = pair ? a : a - 1u;
-    sel = !pair;
-    use_first = !pair;
-  } else {
-    const uint32_t k = ky ^ kz;
-    const uint32_t i0 = (gx ^ k) & (L.size - 1u);
-    lo = i0 & ~1u;
-    sel = i0 & 1u;
-    use_extra = gx & 1u;
-    i1 = ((gx + 1u) ^ k) & (L.size - 1u);
+// Vertex copies.  The encoder reads the coarse levels from copies of its own,
+// laid out by grid vertex, so that the entries of corners x and x + 1 always
+// lie side by side: one 8-byte load per row with no wrap, parity or selects,
+// and one kind of arithmetic for all four lane groups.
+//  * dense levels: entry t of the copy is entry t mod size of the level, up to
+//    the largest index a corner forms (x, y, z <= res);
+//  * hashed levels: vertex (x, y, z), x, y, z <= res, at x + y s + z s^2 with
+//    s = res + 1, holds the entry its hash names.
+// Dense levels are always copied (their size again); hashed ones where that
+// makes a quad of levels uniform and the level's vertices fit in
+// COPY_MAX_ENTRIES (16 MiB): for 2^19 and 2^21 entries and 16..2048 cells the
+// levels up to 7, 24 MiB in all.  Finer levels grow eightfold per doubling
+// while their hashed form stays at the table size.
+// Measured (1920x1080, 44 samples per pixel, with the straight-line quads
+// below): the full-render network 11.35 -> 10.54 ms, 641 -> 500 VALU and 30 ->
+// 26 vector-memory instructions per 16 samples; a refill's frame 30.5 -> 29.3.
+static const int64_t COPY_MAX_ENTRIES = (int64_t)1 << 22;
+
+static int64_t copy_entries(const GridLevel& L, bool dense) {
+  const int64_t r = L.res, s = dense ? r : r + 1;
+  return (r + r * s + r * s * s + 2 + 7) / 8 * 8;  // the last row's pair, and a multiple of 32 bytes
+}
+
+int64_t plan_copies(GridParams& g, int64_t n_entries) {
+  g.copy_mask = g.quad_copy = g.quad_hash = 0;
+  int64_t extra = 0;
+  for (int j = 0; j < 4; j++) {
+    bool all = true;
+    for (int l = 4 * j; l < 4 * j + 4; l++) {
+      const bool dense = (g.dense_mask >> l) & 1u;
+      all = all && (dense || copy_entries(g.lv[l], false) <= COPY_MAX_ENTRIES);
+    }
+    for (int l = 4 * j; l < 4 * j + 4; l++) {
+      const GridLevel& L = g.lv[l];
+      const bool dense = (g.dense_mask >> l) & 1u;
+      EncLevel& E = g.enc[l];
+      E.scale = L.scale;
+      if (all || dense) {
+        const uint32_t s = dense ? L.res : L.res + 1u;
+        E.ya = 4u * s;
+        E.za = 4u * s * s;
+        E.off = (uint32_t)(4 * (n_entries + extra));
+        E.mask = 0;
+        g.copy_mask |= 1u << l;
+        extra += copy_entries(L, dense);
+      } else {
+        E.ya = 4u * 2654435761u;
+        E.za = 4u * 805459861u;
+        E.off = 4u * L.offset;
+        E.mask = 4u * (L.size - 1u);
+      }
+    }
+    const uint32_t q = (g.copy_mask >> (4 * j)) & 15u;
+    if (q == 15u) g.quad_copy |= 1u << j;
+    if (q == 0u) g.quad_hash |= 1u << j;
   }
-  uint2 v;
-  __builtin_memcpy(&v, tl + lo, sizeof(v));
-  uint32_t extra = 0u;
-  if (use_extra) extra = tl[i1];
-  e0 = sel ? v.y : v.x;
-  e1 = use_first ? L.first : (use_extra ? extra : (sel ? v.x : v.y));
+  return extra;
+}
+
+// blockIdx.y: level
+__global__ __launch_bounds__(256) void k_fill_copies(GridParams gp, uint32_t* __restrict__ table) {
+  const int l = blockIdx.y;
+  if (!((gp.copy_mask >> l) & 1u)) return;
+  const GridLevel L = gp.lv[l];
+  const EncLevel E = gp.enc[l];
+  const bool dense = (gp.dense_mask >> l) & 1u;
+  const uint32_t s = E.ya / 4u, n = L.res + L.res * s + L.res * s * s + 2u;
+  uint32_t* out = table + E.off / 4u;
+  const uint32_t* in = table + L.offset;
+  for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) {
+    uint32_t i;
+    if (dense) {
+      i = t % L.size;
+    } else {
+      const uint32_t x = t % s, y = t / s % s, z = t / (s * s);
+      i = (x ^ (y * 2654435761u) ^ (z * 805459861u)) & (L.size - 1u);
+    }
+    out[t] = in[i];
+  }
+}
+void fill_copies(const GridParams& g, uint32_t* table) {
+  if (!g.copy_mask) return;
+  hipLaunchKernelGGL(k_fill_copies, dim3(2048, MAX_LEVELS), dim3(256), 0, 0, g, table);
+  FVC_HIP(hipGetLastError());
+  FVC_HIP(hipStreamSynchronize(0));
+}
+
+// The table as a buffer: 32-bit byte offsets, and a lane whose offset lies
+// past the end reads 0 without a memory access, so a load that only some lanes
+// need is no branch.
+typedef __amdgpu_buffer_rsrc_t TableBuf;
+static const uint32_t NO_LOAD = 0xffffffffu;
+__device__ __forceinline__ TableBuf table_buf(const uint32_t* table, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(table), 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ uint32_t ld1(TableBuf t, uint32_t b) {
+  return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(t, (int)b, 0, 0);
+}
+__device__ __forceinline__ uint2 ld2(TableBuf t, uint32_t b) {  // 4-byte aligned
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  const u2 v = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(t, (int)b, 0, 0));
+  return make_uint2(v.x, v.y);
 }
 
 // Features of levels g, g+4, g+8, g+12 at p (clamped to [0,1]^3) -> f[8]
 // (f[2j], f[2j+1] = level 4j+g).  With this assignment the four lane groups
-// of a wave work on levels 4j..4j+3 together, which are either all dense,
-// all hashed, or (one quad at most) mixed: the first two take wave-uniform
-// branches.  Per level the y / z index terms of both corners are formed once
-// (24-bit products for dense levels, which stay below 2^24); each row of
-// corners x, x + 1 then costs one add or xor, the reduction to the level's
-// entries and (mostly) one 8-byte load (row_pair).
+// of a wave work on levels 4j..4j+3 together, which are either all copied,
+// all hashed, or (other growth factors) mixed.  KIND 1: quads 0 and 1 copied,
+// 2 and 3 hashed (2^19 and 2^21 entries, 16..2048 cells) -- straight-line
+// code, in which every gather is in flight before the first wait; KIND 0: any
+// layout, by wave-uniform branches.  Per level the y / z index terms of both
+// corners are formed once; each row of corners x, x + 1 then costs an add
+// (copied) or a few xors (hashed).
 //
-// HASHED_PAIRS: hashed levels read their rows with row_pair as well (the
-// render kernels); otherwise they, and the mixed quad, read every corner
-// with a load of its own (the fill's latents kernel, whose spatially
-// coherent samples run faster that way).
-template <bool HASHED_PAIRS>
-__device__ __forceinline__ void encode_quads(const GridLevel* __restrict__ lv, const GridParams& gp,
-                                            const uint32_t* __restrict__ table, V3 p, int g, float* f) {
+// Hashed rows (the level's size is a power of two): for even x, x and x + 1
+// differ in bit 0 only, so their entries form the aligned pair holding entry
+// i0; for odd x corner x + 1 is a load of its own (even lanes: NO_LOAD).
+//
+// HASHED_PAIRS: hashed levels read their rows as such pairs (the render
+// kernels); otherwise every corner with a load of its own (the fill's latents
+// kernel, whose spatially coherent samples run faster that way).
+enum { Q_COPY = 0, Q_HASH = 1, Q_MIXED = 2 };
+struct QuadRaw {       // a quad's loads, before selection
+  uint2 v[4];          // the rows' pairs (single loads: corners 2c, 2c + 1)
+  uint32_t extra[4];   // hashed, odd x: corner x + 1
+  bool sel[4];         // hashed: corner x is the pair's second word
+  bool odd;
+};
+template <bool HASHED_PAIRS, int Q>
+__device__ __forceinline__ void quad_loads(const EncLevel& L, bool hashed, TableBuf table, uint32_t gx, uint32_t gy,
+                                           uint32_t gz, QuadRaw& r) {
+  const uint32_t x0 = 4u * gx;
+  r.odd = false;
+  if constexpr (Q == Q_COPY) {
+    const uint32_t y0 = __umul24(gy, L.ya) + x0, z0 = __umul24(gz, L.za) + L.off;
+    const uint32_t yy[2] = {y0, y0 + L.ya}, zz[2] = {z0, z0 + L.za};
+#pragma unroll
+    for (int c = 0; c < 4; c++) r.v[c] = ld2(table, yy[c & 1] + zz[c >> 1]);
+  } else {
+    const uint32_t y0 = gy * L.ya, z0 = gz * L.za;
+    const uint32_t yy[2] = {y0, y0 + L.ya}, zz[2] = {z0, z0 + L.za};
+    if constexpr (Q == Q_HASH && !HASHED_PAIRS) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const uint32_t k = yy[c & 1] ^ zz[c >> 1];
+        r.v[c].x = ld1(table, ((x0 ^ k) & L.mask) + L.off);
+        r.v[c].y = ld1(table, (((x0 + 4u) ^ k) & L.mask) + L.off);
+      }
+    } else {
+      // mixed: lanes of copied levels read at the sum, without a partner's load
+      if (Q == Q_HASH) hashed = true;
+      r.odd = hashed && (gx & 1u);
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const uint32_t k = yy[c & 1] ^ zz[c >> 1];
+        const uint32_t i0 = (x0 ^ k) & L.mask;
+        r.v[c] = ld2(table, (hashed ? i0 & ~4u : x0 + yy[c & 1] + zz[c >> 1]) + L.off);
+        r.extra[c] = ld1(table, r.odd ? (((x0 + 4u) ^ k) & L.mask) + L.off : NO_LOAD);
+        r.sel[c] = hashed && (i0 & 4u);
+      }
+    }
+  }
+}
+template <bool HASHED_PAIRS, int Q>
+__device__ __forceinline__ void quad_entries(const QuadRaw& r, uint32_t (&ent)[8]) {
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    if constexpr (Q == Q_COPY || (Q == Q_HASH && !HASHED_PAIRS)) {
+      ent[2 * c] = r.v[c].x;
+      ent[2 * c + 1] = r.v[c].y;
+    } else {
+      ent[2 * c] = r.sel[c] ? r.v[c].y : r.v[c].x;
+      ent[2 * c + 1] = r.odd ? r.extra[c] : (r.sel[c] ? r.v[c].x : r.v[c].y);
+    }
+  }
+}
+template <bool HASHED_PAIRS, int KIND>
+__device__ __forceinline__ void encode_quads(const EncLevel* __restrict__ lv, const GridParams& gp, TableBuf table,
+                                            V3 p, int g, float* f) {
   const float px = fminf_(fmaxf_(p.x, 0.0f), 1.0f);
   const float py = fminf_(fmaxf_(p.y, 0.0f), 1.0f);
   const float pz = fminf_(fmaxf_(p.z, 0.0f), 1.0f);
   uint32_t ent[4][8];
+  QuadRaw raw[4];
   float wx[4], wy[4], wz[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int l = 4 * j + g;
-    const GridLevel L = lv[l];
+    const EncLevel L = lv[l];
     const float ax = px * L.scale + 0.5f, ay = py * L.scale + 0.5f, az = pz * L.scale + 0.5f;
     const float fx = floorf(ax), fy = floorf(ay), fz = floorf(az);
     const uint32_t gx = (uint32_t)(int)fx, gy = (uint32_t)(int)fy, gz = (uint32_t)(int)fz;
     wx[j] = ax - fx; wy[j] = ay - fy; wz[j] = az - fz;
-    const uint32_t* tl = table + L.offset;
-    // the four (y, z) rows of the cell, corners x and x + 1 each
-    auto rows = [&](bool dense, bool pairs) {
-      const uint32_t y0 = dense ? __umul24(gy, L.res) : gy * 2654435761u;
-      const uint32_t z0 = dense ? __umul24(gz, L.res2) : gz * 805459861u;
-      const uint32_t yy[2] = {y0, y0 + (dense ? L.res : 2654435761u)};
-      const uint32_t zz[2] = {z0, z0 + (dense ? L.res2 : 805459861u)};
-#pragma unroll
-      for (int c = 0; c < 8; c += 2) {
-        const uint32_t ky = yy[(c >> 1) & 1], kz = zz[c >> 2];
-        if (pairs) {
-          row_pair(tl, L, dense, gx, ky, kz, ent[j][c], ent[j][c + 1]);
-        } else {
-#pragma unroll
-          for (int o = 0; o < 2; o++) {
-            const uint32_t x = gx + o, ta = x + ky + kz, th = (x ^ ky ^ kz) & (L.size - 1u);
-            ent[j][c + o] = tl[dense ? min(ta, ta - L.size) : th];  // ta < 2 * size
-          }
-        }
-      }
-    };
-    if ((gp.quad_dense >> j) & 1u) rows(true, true);
-    else if ((gp.quad_hash >> j) & 1u) rows(false, HASHED_PAIRS);
-    else rows((gp.dense_mask >> l) & 1u, HASHED_PAIRS);
+    if constexpr (KIND == 1) {
+      if (j < 2) quad_loads<HASHED_PAIRS, Q_COPY>(L, false, table, gx, gy, gz, raw[j]);
+      else quad_loads<HASHED_PAIRS, Q_HASH>(L, true, table, gx, gy, gz, raw[j]);
+    } else if ((gp.quad_copy >> j) & 1u) {
+      quad_loads<HASHED_PAIRS, Q_COPY>(L, false, table, gx, gy, gz, raw[j]);
+      quad_entries<HASHED_PAIRS, Q_COPY>(raw[j], ent[j]);
+    } else if ((gp.quad_hash >> j) & 1u) {
+      quad_loads<HASHED_PAIRS, Q_HASH>(L, true, table, gx, gy, gz, raw[j]);
+      quad_entries<HASHED_PAIRS, Q_HASH>(raw[j], ent[j]);
+    } else {
+      quad_loads<HASHED_PAIRS, Q_MIXED>(L, !((gp.copy_mask >> l) & 1u), table, gx, gy, gz, raw[j]);
+      quad_entries<HASHED_PAIRS, Q_MIXED>(raw[j], ent[j]);
+    }
   }
 #pragma unroll
   for (int j = 0; j < 4; j++) {
+    if constexpr (KIND == 1) {
+      if (j < 2) quad_entries<HASHED_PAIRS, Q_COPY>(raw[j], ent[j]);
+      else quad_entries<HASHED_PAIRS, Q_HASH>(raw[j], ent[j]);
+    }
     const float ux = 1.0f - wx[j], uy = 1.0f - wy[j], uz = 1.0f - wz[j];
     const float wxy[4] = {ux * uy, wx[j] * uy, ux * wy[j], wx[j] * wy[j]};
     float a0 = 0.0f, a1 = 0.0f;
@@ -203,15 +316,12 @@ __device__ __forceinline__ void encode_quads(const GridLevel* __restrict__ lv, c
     f[2 * j + 1] = a1;
   }
 }
+// the layout that encode_quads<., 1> takes
+static int enc_kind(const GridParams& g) { return g.quad_copy == 3u && g.quad_hash == 12u ? 1 : 0; }
 
-// the block's copy of the level table, with each level's entry 0
-__device__ __forceinline__ void load_levels(const GridParams& gp, const uint32_t* __restrict__ table,
-                                            GridLevel* lv) {
-  if (threadIdx.x < MAX_LEVELS) {
-    GridLevel L = gp.lv[threadIdx.x];
-    if ((int)threadIdx.x < gp.n_levels) L.first = table[L.offset];
-    lv[threadIdx.x] = L;
-  }
+// the block's copy of the level table
+__device__ __forceinline__ void load_levels(const GridParams& gp, EncLevel* lv) {
+  if (threadIdx.x < MAX_LEVELS) lv[threadIdx.x] = gp.enc[threadIdx.x];
   __syncthreads();
 }
 
@@ -233,18 +343,20 @@ __device__ __forceinline__ uint2 pack_h4(_Float16 a, _Float16 b, _Float16 c, _Fl
 // bits) per sample and dir is the per-pixel SH table (sh4_all, 32 bytes per
 // pixel, written by the marcher at the ray's first launch) instead of a
 // direction per sample.
-template <bool HEAD, int P, int TILES, bool PIX = false>
+template <bool HEAD, int P, int TILES, int KIND, bool PIX = false>
 __global__ __launch_bounds__(NET_BLOCK) void k_network(const float* __restrict__ pos, const float* __restrict__ dir,
                                                        int64_t n, const uint32_t* __restrict__ table,
+                                                       uint32_t table_bytes,
                                                        const typename Mx<P>::T* __restrict__ frags, GridParams gp,
                                                        MlpScales sc, uint2* __restrict__ out_h4,
                                                        uint2* __restrict__ out16, const int* __restrict__ n_dev) {
   // n_dev: sample count written by an earlier kernel (n is then its bound)
   if (n_dev) n = *n_dev;
   if ((int64_t)blockIdx.x * (NET_BLOCK / 64) * 16 * TILES >= n) return;
-  __shared__ GridLevel lv[MAX_LEVELS];
+  __shared__ EncLevel lv[MAX_LEVELS];
   __shared__ typename Mx<P>::T wl[N_NET_FRAGS * 64];
-  load_levels(gp, table, lv);
+  const TableBuf tbuf = table_buf(table, table_bytes);
+  load_levels(gp, lv);
   stage_frags(frags, wl, N_NET_FRAGS);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -277,7 +389,7 @@ __global__ __launch_bounds__(NET_BLOCK) void k_network(const float* __restrict__
     }
 #pragma unroll
     for (int t = 0; t < TILES; t++) {
-      encode_quads<HEAD>(lv, gp, table, pv[t], g, f[t]);
+      encode_quads<HEAD, KIND>(lv, gp, tbuf, pv[t], g, f[t]);
       // pinned here (after the gathers are issued): otherwise the load sinks
       // to its use after the density MLP and waits there on its own
       if constexpr (HEAD && PIX) {
@@ -357,17 +469,19 @@ __global__ __launch_bounds__(NET_BLOCK) void k_head(const uint16_t* __restrict__
 // di: the first latent is log sigma (the first head's latent row 0 is then
 // a zero-weight row replaced here).  FL: first-head hidden layers.
 // PIX (FULL only): the renderer's sample stream as in k_network.
-template <bool FULL, int TILES, int FL, bool PIX = false>
+template <bool FULL, int TILES, int FL, int KIND, bool PIX = false>
 __global__ __launch_bounds__(NET_BLOCK) void k_network_vd(const float* __restrict__ pos, const float* __restrict__ dir,
                                                           int64_t n, const uint32_t* __restrict__ table,
+                                                          uint32_t table_bytes,
                                                           const h8* __restrict__ frags, GridParams gp, int di,
                                                           int freq_on, uint2* __restrict__ out,
                                                           const int* __restrict__ n_dev) {
   if (n_dev) n = *n_dev;
   if ((int64_t)blockIdx.x * (NET_BLOCK / 64) * 16 * TILES >= n) return;
-  __shared__ GridLevel lv[MAX_LEVELS];
+  __shared__ EncLevel lv[MAX_LEVELS];
   __shared__ h8 wl[N_VD_NET_FRAGS * 64];
-  load_levels(gp, table, lv);
+  const TableBuf tbuf = table_buf(table, table_bytes);
+  load_levels(gp, lv);
   stage_frags(frags, wl, FULL ? N_VD_NET_FRAGS : VD_HA);
   __syncthreads();
   const MlpScales sc{{1.0f, 1.0f, 1.0f, 1.0f, 1.0f}, 1.0f};
@@ -399,7 +513,7 @@ __global__ __launch_bounds__(NET_BLOCK) void k_network_vd(const float* __restric
     }
 #pragma unroll
     for (int t = 0; t < TILES; t++) {
-      encode_quads<FULL>(lv, gp, table, pv[t], g, f[t]);
+      encode_quads<FULL, KIND>(lv, gp, tbuf, pv[t], g, f[t]);
       // pinned here (after the gathers are issued), as in k_network
       if constexpr (PIX) {
         shq[t] = reinterpret_cast<const uint2*>(dir)[(int64_t)px[t] * 4 + g];
@@ -478,16 +592,19 @@ __global__ __launch_bounds__(NET_BLOCK) void k_head_vd(const uint16_t* __restric
 }
 
 // encoding alone: 32 halves per sample (thread per sample)
-__global__ void k_encode(const float* __restrict__ pos, int64_t n, const uint32_t* __restrict__ table, GridParams gp,
+template <int KIND>
+__global__ void k_encode(const float* __restrict__ pos, int64_t n, const uint32_t* __restrict__ table,
+                         uint32_t table_bytes, GridParams gp,
                          uint16_t* __restrict__ out32) {
-  __shared__ GridLevel lv[MAX_LEVELS];
-  load_levels(gp, table, lv);
+  __shared__ EncLevel lv[MAX_LEVELS];
+  const TableBuf tbuf = table_buf(table, table_bytes);
+  load_levels(gp, lv);
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const V3 p = {pos[3 * s], pos[3 * s + 1], pos[3 * s + 2]};
   for (int q = 0; q < 4; q++) {
     float f[8];
-    encode_quads<true>(lv, gp, table, p, q, f);
+    encode_quads<true, KIND>(lv, gp, tbuf, p, q, f);
     for (int j = 0; j < 4; j++)
       for (int k = 0; k < 2; k++)
         out32[s * 32 + 2 * (4 * j + q) + k] = __builtin_bit_cast(uint16_t, (_Float16)f[2 * j + k]);
@@ -531,13 +648,16 @@ void launch_network_full_ex(const Model& m, const float* pos, const float* dir, 
     launch_network_full_vd(m, pos, dir, pix, n, out_h4, s, n_dev, rows);
     return;
   }
-#define L3(P, TL, PX)                                                                                              \
-  hipLaunchKernelGGL((k_network<true, P, TL, PX>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), 0, \
-                     s, pos, dir, n, m.table.as<uint32_t>(), m.frags.as<typename Mx<P>::T>(), m.grid, m.mlp_scales,  \
+#define L4(P, TL, KD, PX)                                                                                          \
+  hipLaunchKernelGGL((k_network<true, P, TL, KD, PX>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), 0, \
+                     s, pos, dir, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<typename Mx<P>::T>(), m.grid, m.mlp_scales,  \
                      (uint2*)out_h4, (uint2*)nullptr, n_dev)
-#define L2(P, TL)          \
-  if (pix) { L3(P, TL, true); } \
-  else { L3(P, TL, false); }
+#define L3(P, TL, KD)              \
+  if (pix) { L4(P, TL, KD, true); } \
+  else { L4(P, TL, KD, false); }
+#define L2(P, TL)                        \
+  if (enc_kind(m.grid)) { L3(P, TL, 1) } \
+  else { L3(P, TL, 0) }
 #define L(P)                       \
   if (rows == 64) { L2(P, 4); }    \
   else if (rows == 32) { L2(P, 2); } \
@@ -546,16 +666,20 @@ void launch_network_full_ex(const Model& m, const float* pos, const float* dir, 
 #undef L
 #undef L2
 #undef L3
+#undef L4
   FVC_HIP(hipGetLastError());
 }
 void launch_network_latents(const Model& m, const float* pos, int64_t n, uint16_t* out16, hipStream_t s, int rows,
                             const int* n_dev, uint16_t* log_sigma) {
   if (m.net.split_head) throw Error(FVC_E_UNSUPPORTED, "split models need the initial view direction");
   if (n <= 0) return;
-#define L2(P, TL)                                                                                                 \
-  hipLaunchKernelGGL((k_network<false, P, TL>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), 0, s, \
-                     pos, (const float*)nullptr, n, m.table.as<uint32_t>(), m.frags.as<typename Mx<P>::T>(), m.grid, \
+#define L3(P, TL, KD)                                                                                             \
+  hipLaunchKernelGGL((k_network<false, P, TL, KD>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), 0, s, \
+                     pos, (const float*)nullptr, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<typename Mx<P>::T>(), m.grid, \
                      m.mlp_scales, (uint2*)log_sigma, (uint2*)out16, n_dev)
+#define L2(P, TL)                       \
+  if (enc_kind(m.grid)) { L3(P, TL, 1); } \
+  else { L3(P, TL, 0); }
 #define L(P)                       \
   if (rows == 64) { L2(P, 4); }    \
   else if (rows == 32) { L2(P, 2); } \
@@ -563,6 +687,7 @@ void launch_network_latents(const Model& m, const float* pos, int64_t n, uint16_
   FVC_BY_PREC(m, L)
 #undef L
 #undef L2
+#undef L3
   FVC_HIP(hipGetLastError());
 }
 void launch_network_head(const Model& m, const uint16_t* hin16, const float* dir, int64_t n, uint32_t* out_h4,
@@ -580,13 +705,16 @@ void launch_network_full_vd(const Model& m, const float* pos, const float* dir, 
                             uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows) {
   if (n <= 0) return;
   const int di = m.net.first_latent_is_density, fq = m.net.freq_encoding_degree > 0;
-#define L2(TL, FL, PX)                                                                                            \
-  hipLaunchKernelGGL((k_network_vd<true, TL, FL, PX>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))),             \
-                     dim3(NET_BLOCK), 0, s, pos, dir, n, m.table.as<uint32_t>(), m.frags.as<h8>(), m.grid, di, fq,  \
+#define L3(TL, FL, KD, PX)                                                                                        \
+  hipLaunchKernelGGL((k_network_vd<true, TL, FL, KD, PX>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))),             \
+                     dim3(NET_BLOCK), 0, s, pos, dir, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<h8>(), m.grid, di, fq,  \
                      (uint2*)out_h4, n_dev)
-#define L(TL, FL)                \
-  if (pix) { L2(TL, FL, true); } \
-  else { L2(TL, FL, false); }
+#define L2(TL, FL, KD)               \
+  if (pix) { L3(TL, FL, KD, true); } \
+  else { L3(TL, FL, KD, false); }
+#define L(TL, FL)                        \
+  if (enc_kind(m.grid)) { L2(TL, FL, 1) } \
+  else { L2(TL, FL, 0) }
   if (m.net.first_head_n_hidden_layers == 2) {
     if (rows == 64) { L(4, 2); } else if (rows == 32) { L(2, 2); } else { L(1, 2); }
   } else {
@@ -594,22 +722,27 @@ void launch_network_full_vd(const Model& m, const float* pos, const float* dir, 
   }
 #undef L
 #undef L2
+#undef L3
   FVC_HIP(hipGetLastError());
 }
 void launch_network_latents_vd(const Model& m, const float* pos, const float* init_dir, int64_t n, uint16_t* out16,
                                hipStream_t s, int rows, const int* n_dev) {
   if (n <= 0) return;
   const int di = m.net.first_latent_is_density, fq = m.net.freq_encoding_degree > 0;
-#define L(TL, FL)                                                                                               \
-  hipLaunchKernelGGL((k_network_vd<false, TL, FL>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), \
-                     0, s, pos, init_dir, n, m.table.as<uint32_t>(), m.frags.as<h8>(), m.grid, di, fq,            \
+#define L2(TL, FL, KD)                                                                                          \
+  hipLaunchKernelGGL((k_network_vd<false, TL, FL, KD>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), \
+                     0, s, pos, init_dir, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<h8>(), m.grid, di, fq,            \
                      (uint2*)out16, n_dev)
+#define L(TL, FL)                          \
+  if (enc_kind(m.grid)) { L2(TL, FL, 1); } \
+  else { L2(TL, FL, 0); }
   if (m.net.first_head_n_hidden_layers == 2) {
     if (rows == 64) { L(4, 2); } else if (rows == 32) { L(2, 2); } else { L(1, 2); }
   } else {
     if (rows == 64) { L(4, 1); } else if (rows == 32) { L(2, 1); } else { L(1, 1); }
   }
 #undef L
+#undef L2
   FVC_HIP(hipGetLastError());
 }
 void launch_network_head_vd(const Model& m, const uint16_t* head_in16, const float* pos, const float* dir,
@@ -623,8 +756,8 @@ void launch_network_head_vd(const Model& m, const uint16_t* head_in16, const flo
 
 void launch_network_encode(const Model& m, const float* pos, int64_t n, uint16_t* out32, hipStream_t s) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_encode, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, pos, n, m.table.as<uint32_t>(),
-                     m.grid, out32);
+  hipLaunchKernelGGL(enc_kind(m.grid) ? k_encode<1> : k_encode<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, pos, n, m.table.as<uint32_t>(),
+                     (uint32_t)m.table.bytes, m.grid, out32);
   FVC_HIP(hipGetLastError());
 }
 
