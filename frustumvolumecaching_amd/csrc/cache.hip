@@ -1504,7 +1504,7 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       h.march = P.end(ev, s, "cache_march");
       ev = P.begin(s);
       launch_network_full_pix(m, r.s_pos.as<float4>(), r.ray_sh.as<uint4>(), n_bound, r.s_out.as<uint32_t>(), s,
-                              ctl + CTL_R, r.mlp_rows);
+                              ctl + CTL_R, r.mlp_rows, false);
       h.net = P.end(ev, s, "network_resample");
       ev = P.begin(s);
 #define L2(P, F8)                                                                                                    \

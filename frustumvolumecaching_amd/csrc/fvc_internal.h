@@ -170,11 +170,12 @@ void nerfacc_read_data(const std::string& dir, const NerfaccExport& ex, uint16_t
 void launch_network_full(const Model& m, const float* pos, const float* dir, int64_t n, uint32_t* out_h4,
                          hipStream_t s, const int* n_dev = nullptr, int rows = 16);
 // the renderer's sample stream: pos4 = (x, y, z, pixel index bits) per
-// sample, ray_sh the per-pixel SH table (sh4_all)
+// sample, ray_sh the per-pixel SH table (sh4_all); near_bound: the count on the
+// device is usually near n
 void launch_network_full_pix(const Model& m, const float4* pos4, const uint4* ray_sh, int64_t n, uint32_t* out_h4,
-                             hipStream_t s, const int* n_dev, int rows);
+                             hipStream_t s, const int* n_dev, int rows, bool near_bound);
 void launch_network_full_ex(const Model& m, const float* pos, const float* dir, bool pix, int64_t n,
-                            uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows);
+                            uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows, int64_t cap);
 // log_sigma (optional): row 0 of each sample once more, as a compact half array
 void launch_network_latents(const Model& m, const float* pos, int64_t n, uint16_t* out16, hipStream_t s,
                             int rows = 16, const int* n_dev = nullptr, uint16_t* log_sigma = nullptr);
@@ -185,7 +186,7 @@ void launch_network_encode(const Model& m, const float* pos, int64_t n, uint16_t
 // dir), latents with the initial view direction init_dir ([8 head latents,
 // log sigma] per sample), the custom head alone
 void launch_network_full_vd(const Model& m, const float* pos, const float* dir, bool pix, int64_t n,
-                            uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows);
+                            uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows, int64_t cap);
 void launch_network_latents_vd(const Model& m, const float* pos, const float* init_dir, int64_t n, uint16_t* out16,
                                hipStream_t s, int rows, const int* n_dev = nullptr);
 void launch_network_head_vd(const Model& m, const uint16_t* head_in16, const float* pos, const float* dir,

@@ -335,6 +335,30 @@ __device__ __forceinline__ uint2 pack_h4(_Float16 a, _Float16 b, _Float16 c, _Fl
   return v;
 }
 
+// The order in which a launch's blocks take its n samples.  Block b runs on
+// XCD b % 8, and the XCDs share no L2, so runs of `chunk` consecutive units (a
+// unit: `per` samples, one group per wave) go to one XCD: neighbouring rays
+// then find each other's table lines in its L2.  Small launches spread over
+// all XCDs.  Returns the block's first unit; its next ones follow at
+// gridDim.x (net_grid: a multiple of 8 chunks).  A larger grid keeps the units
+// in flight closer together but stages the weights more often and costs more
+// idle blocks where n falls short of the launch's bound.
+// Measured (us, frames of the unbounded scene; 48 samples per pixel): without
+// chunks 1920x1080 13270, 1280x720 6900, 12 views 31550; chunks of 4 / 16 /
+// 32 / 64 / 128 units 12770 / 12110 / 12020 / 11990 / 12010 at 1920x1080
+// (L2 misses 464 -> 118 M, 5.1 -> 1.3 a sample), 12 views 24600 with 64; grids
+// of 16384 / 32768 / 65536 blocks: 11990 / 11800 / 11730, 12 views 24570 /
+// 23150 / 22040, but 800x800 of the small scene, many launches far below
+// their bound, 6765 / 6940 / 7140, and a refill 23120 / 23350 / 23950.  A grid
+// of the resident blocks only, striding on, drifts apart: 13000.
+static const int NET_CHUNK = 64;
+static const int NET_BLOCKS_FULL = 32768, NET_BLOCKS = 16384;  // full renders; launches far below their bound
+__device__ __forceinline__ int64_t net_first_unit(int64_t n, int per) {
+  const int shift = n >= (int64_t)64 * NET_CHUNK * per ? 6 : (n >= (int64_t)64 * 8 * per ? 3 : 0);  // chunk 64, 8, 1
+  const int b = blockIdx.x, m = (8 << shift) - 1;
+  return (b & ~m) + ((b & 7) << shift) + ((b & m) >> 3);
+}
+
 // HEAD: full inference -> half4 (r, g, b, log sigma) per sample
 // !HEAD: inferenceLatents -> 16 halves per sample
 // TILES: 16-sample MFMA tiles per wave and loop iteration (MLP rows per
@@ -352,7 +376,8 @@ __global__ __launch_bounds__(NET_BLOCK) void k_network(const float* __restrict__
                                                        uint2* __restrict__ out16, const int* __restrict__ n_dev) {
   // n_dev: sample count written by an earlier kernel (n is then its bound)
   if (n_dev) n = *n_dev;
-  if ((int64_t)blockIdx.x * (NET_BLOCK / 64) * 16 * TILES >= n) return;
+  const int64_t unit = net_first_unit(n, NET_BLOCK / 64 * 16 * TILES);
+  if (unit * (NET_BLOCK / 64) * 16 * TILES >= n) return;
   __shared__ EncLevel lv[MAX_LEVELS];
   __shared__ typename Mx<P>::T wl[N_NET_FRAGS * 64];
   const TableBuf tbuf = table_buf(table, table_bytes);
@@ -362,8 +387,7 @@ __global__ __launch_bounds__(NET_BLOCK) void k_network(const float* __restrict__
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int64_t n_groups = (n + 16 * TILES - 1) / (16 * TILES);
-  for (int64_t grp = (int64_t)blockIdx.x * (NET_BLOCK / 64) + wave; grp < n_groups;
-       grp += (int64_t)gridDim.x * (NET_BLOCK / 64)) {
+  for (int64_t grp = unit * (NET_BLOCK / 64) + wave; grp < n_groups; grp += (int64_t)gridDim.x * (NET_BLOCK / 64)) {
     const int li = opaque(lane);
     int64_t s[TILES], sl[TILES];
     bool valid[TILES];
@@ -477,7 +501,8 @@ __global__ __launch_bounds__(NET_BLOCK) void k_network_vd(const float* __restric
                                                           int freq_on, uint2* __restrict__ out,
                                                           const int* __restrict__ n_dev) {
   if (n_dev) n = *n_dev;
-  if ((int64_t)blockIdx.x * (NET_BLOCK / 64) * 16 * TILES >= n) return;
+  const int64_t unit = net_first_unit(n, NET_BLOCK / 64 * 16 * TILES);
+  if (unit * (NET_BLOCK / 64) * 16 * TILES >= n) return;
   __shared__ EncLevel lv[MAX_LEVELS];
   __shared__ h8 wl[N_VD_NET_FRAGS * 64];
   const TableBuf tbuf = table_buf(table, table_bytes);
@@ -488,8 +513,7 @@ __global__ __launch_bounds__(NET_BLOCK) void k_network_vd(const float* __restric
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int64_t n_groups = (n + 16 * TILES - 1) / (16 * TILES);
-  for (int64_t grp = (int64_t)blockIdx.x * (NET_BLOCK / 64) + wave; grp < n_groups;
-       grp += (int64_t)gridDim.x * (NET_BLOCK / 64)) {
+  for (int64_t grp = unit * (NET_BLOCK / 64) + wave; grp < n_groups; grp += (int64_t)gridDim.x * (NET_BLOCK / 64)) {
     const int li = opaque(lane);
     int64_t s[TILES], sl[TILES];
     bool valid[TILES];
@@ -611,12 +635,15 @@ __global__ void k_encode(const float* __restrict__ pos, int64_t n, const uint32_
   }
 }
 
+// blocks for up to n samples of `per` a unit (net_first_unit)
+static int net_grid(int64_t n, int per, int64_t cap) {
+  const int64_t units = std::max<int64_t>(1, std::min<int64_t>((n + per - 1) / per, cap)), m = 8 * NET_CHUNK;
+  return (int)((units + m - 1) / m * m);
+}
+// blocks of the head kernels (given inputs, no table), grid-stride beyond
 static int grid_for(int64_t n_groups) {
   const int64_t waves = n_groups;
   int64_t blocks = (waves + NET_BLOCK / 64 - 1) / (NET_BLOCK / 64);
-  // 16384 blocks (64 per CU), grid-stride beyond: measured on the 1080p path
-  // against 4096 - 65536 (more blocks help the full render; the resample
-  // launches, sized by a bound, pay for blocks that find no work)
   const int64_t cap = 16384;
   if (blocks > cap) blocks = cap;
   if (blocks < 1) blocks = 1;
@@ -634,30 +661,32 @@ static int grid_for(int64_t n_groups) {
 
 void launch_network_full(const Model& m, const float* pos, const float* dir, int64_t n, uint32_t* out_h4,
                          hipStream_t s, const int* n_dev, int rows) {
-  launch_network_full_ex(m, pos, dir, false, n, out_h4, s, n_dev, rows);
+  launch_network_full_ex(m, pos, dir, false, n, out_h4, s, n_dev, rows, NET_BLOCKS);
 }
 void launch_network_full_pix(const Model& m, const float4* pos4, const uint4* ray_sh, int64_t n, uint32_t* out_h4,
-                             hipStream_t s, const int* n_dev, int rows) {
+                             hipStream_t s, const int* n_dev, int rows, bool near_bound) {
   launch_network_full_ex(m, reinterpret_cast<const float*>(pos4), reinterpret_cast<const float*>(ray_sh), true, n,
-                         out_h4, s, n_dev, rows);
+                         out_h4, s, n_dev, rows, near_bound ? NET_BLOCKS_FULL : NET_BLOCKS);
 }
 void launch_network_full_ex(const Model& m, const float* pos, const float* dir, bool pix, int64_t n, uint32_t* out_h4,
-                            hipStream_t s, const int* n_dev, int rows) {
+                            hipStream_t s, const int* n_dev, int rows, int64_t cap) {
   if (n <= 0) return;
   if (m.net.split_head) {
-    launch_network_full_vd(m, pos, dir, pix, n, out_h4, s, n_dev, rows);
+    launch_network_full_vd(m, pos, dir, pix, n, out_h4, s, n_dev, rows, cap);
     return;
   }
 #define L4(P, TL, KD, PX)                                                                                          \
-  hipLaunchKernelGGL((k_network<true, P, TL, KD, PX>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), 0, \
+  hipLaunchKernelGGL((k_network<true, P, TL, KD, PX>), dim3(net_grid(n, NET_BLOCK / 64 * 16 * TL, cap)), dim3(NET_BLOCK), 0, \
                      s, pos, dir, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<typename Mx<P>::T>(), m.grid, m.mlp_scales,  \
                      (uint2*)out_h4, (uint2*)nullptr, n_dev)
-#define L3(P, TL, KD)              \
-  if (pix) { L4(P, TL, KD, true); } \
-  else { L4(P, TL, KD, false); }
-#define L2(P, TL)                        \
-  if (enc_kind(m.grid)) { L3(P, TL, 1) } \
-  else { L3(P, TL, 0) }
+  // A caller's own points (not pix) are scattered and bound by the lines they
+  // touch, not by instructions: the loads of one quad at a time are then as
+  // good or better (1 M random points: fp16 826 us against 841 straight-line,
+  // fp8 835 / 843, bf16x3 838 / 857).
+#define L2(P, TL)                                      \
+  if (!pix) { L4(P, TL, 0, false); }                   \
+  else if (enc_kind(m.grid)) { L4(P, TL, 1, true); }   \
+  else { L4(P, TL, 0, true); }
 #define L(P)                       \
   if (rows == 64) { L2(P, 4); }    \
   else if (rows == 32) { L2(P, 2); } \
@@ -665,7 +694,6 @@ void launch_network_full_ex(const Model& m, const float* pos, const float* dir, 
   FVC_BY_PREC(m, L)
 #undef L
 #undef L2
-#undef L3
 #undef L4
   FVC_HIP(hipGetLastError());
 }
@@ -674,7 +702,7 @@ void launch_network_latents(const Model& m, const float* pos, int64_t n, uint16_
   if (m.net.split_head) throw Error(FVC_E_UNSUPPORTED, "split models need the initial view direction");
   if (n <= 0) return;
 #define L3(P, TL, KD)                                                                                             \
-  hipLaunchKernelGGL((k_network<false, P, TL, KD>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), 0, s, \
+  hipLaunchKernelGGL((k_network<false, P, TL, KD>), dim3(net_grid(n, NET_BLOCK / 64 * 16 * TL, NET_BLOCKS)), dim3(NET_BLOCK), 0, s, \
                      pos, (const float*)nullptr, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<typename Mx<P>::T>(), m.grid, \
                      m.mlp_scales, (uint2*)log_sigma, (uint2*)out16, n_dev)
 #define L2(P, TL)                       \
@@ -702,11 +730,11 @@ void launch_network_head(const Model& m, const uint16_t* hin16, const float* dir
   FVC_HIP(hipGetLastError());
 }
 void launch_network_full_vd(const Model& m, const float* pos, const float* dir, bool pix, int64_t n,
-                            uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows) {
+                            uint32_t* out_h4, hipStream_t s, const int* n_dev, int rows, int64_t cap) {
   if (n <= 0) return;
   const int di = m.net.first_latent_is_density, fq = m.net.freq_encoding_degree > 0;
 #define L3(TL, FL, KD, PX)                                                                                        \
-  hipLaunchKernelGGL((k_network_vd<true, TL, FL, KD, PX>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))),             \
+  hipLaunchKernelGGL((k_network_vd<true, TL, FL, KD, PX>), dim3(net_grid(n, NET_BLOCK / 64 * 16 * TL, cap)),             \
                      dim3(NET_BLOCK), 0, s, pos, dir, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<h8>(), m.grid, di, fq,  \
                      (uint2*)out_h4, n_dev)
 #define L2(TL, FL, KD)               \
@@ -730,7 +758,7 @@ void launch_network_latents_vd(const Model& m, const float* pos, const float* in
   if (n <= 0) return;
   const int di = m.net.first_latent_is_density, fq = m.net.freq_encoding_degree > 0;
 #define L2(TL, FL, KD)                                                                                          \
-  hipLaunchKernelGGL((k_network_vd<false, TL, FL, KD>), dim3(grid_for((n + 16 * TL - 1) / (16 * TL))), dim3(NET_BLOCK), \
+  hipLaunchKernelGGL((k_network_vd<false, TL, FL, KD>), dim3(net_grid(n, NET_BLOCK / 64 * 16 * TL, NET_BLOCKS)), dim3(NET_BLOCK), \
                      0, s, pos, init_dir, n, m.table.as<uint32_t>(), (uint32_t)m.table.bytes, m.frags.as<h8>(), m.grid, di, fq,            \
                      (uint2*)out16, n_dev)
 #define L(TL, FL)                          \

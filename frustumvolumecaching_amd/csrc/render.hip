@@ -590,7 +590,7 @@ void render_full(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       h.march = P.end(ev, s, "march");
       ev = P.begin(s);
       launch_network_full_pix(m, r.s_pos.as<float4>(), r.ray_sh.as<uint4>(), n_bound, r.s_out.as<uint32_t>(), s,
-                              ctl + CTL_R, r.mlp_rows);
+                              ctl + CTL_R, r.mlp_rows, true);
       h.net = P.end(ev, s, "network_full");
       ev = P.begin(s);
       hipLaunchKernelGGL(k_composite, grid, dim3(256), 0, s, ctl, cur, rm.stepsize_info, m.scene.alpha_thre,
@@ -755,7 +755,7 @@ void render_full_noalloc(Renderer& r, const fvc_raymarch_info& rm, uint8_t* rgba
                        pix[cur], entry, alive, t_scr, s_pos, ray_sh, s_t0);
     FVC_HIP(hipGetLastError());
     launch_network_full_pix(m, s_pos, ray_sh, n_bound, reinterpret_cast<uint32_t*>(s_out), s, ctl + CTL_R,
-                            r.mlp_rows);
+                            r.mlp_rows, false);
     hipLaunchKernelGGL(k_composite, grid, dim3(256), 0, s, ctl, cur, rm.stepsize_info, m.scene.alpha_thre, rays[cur],
                        pix[cur], rres[cur], entry, alive, s_out, s_t0, rays[cur ^ 1], pix[cur ^ 1], rres[cur ^ 1],
                        results);

@@ -43,3 +43,24 @@ def test_layouts(oracle_mod, log2_size, base, finest):
     assert_fp16_close(host_f16(lat)[:, :9], ref.latents(p, oracle_mod.EMU16)[:, :9])
     assert_fp16_close(host_f16(out), ref.inference(p, d01, oracle_mod.EMU16))
     model.close()
+
+
+# launches below, at and above the lines between the orders in which the blocks
+# take their samples, and past the largest grid
+@pytest.mark.parametrize("n", [1, 32767, 65537, 262143, 262145, 524289, (1 << 21) + 1, (1 << 22) + 65])
+def test_every_sample_is_taken(n):
+    model = lib.NerfNetwork.from_workload(S.small_plain(8, 8, stepsize_setup=lib.stepsize_setup))
+    period = 4099
+    p = dev(_positions(period, 7))
+    d = torch.full((period, 3), 0.25, device="cuda")
+    at = torch.arange(n, device="cuda") % period
+    got = []
+    for pos, dirs in ((p, d), (p[at].contiguous(), d[at].contiguous())):
+        lat, out = empty((len(pos), 16), torch.int16).fill_(-1), empty((len(pos), 4), torch.int16).fill_(-1)
+        model.inferenceLatents(pos, len(pos), lat)
+        model.inference(pos, dirs, len(pos), out)
+        got.append((lat, out))
+    torch.cuda.synchronize()
+    for one, all_ in zip(*got):
+        assert torch.equal(all_, one[at])
+    model.close()
