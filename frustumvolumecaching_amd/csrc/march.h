@@ -146,18 +146,24 @@ FVC_HD Skip box_skip(int cx, int cy, int cz, int g, int mip, const OccParams& o,
   return Skip{tin, tout};
 }
 
-// grid_occupied_at<128, true> (raymarch_common.h:680-710) for p = o + tm*d.
-// When the answer is "empty" the skip interval of the largest empty box
-// around the cell is stored in sk (left unchanged outside every cascade).
-FVC_HD bool occ_query(V3 p, const OccParams& o, const uint64_t* __restrict__ bf64, const uint32_t* coarse,
-                      const RaySlab& rs, Skip& sk) {
+// grid_occupied_at<128, true> (raymarch_common.h:680-710) in three parts, so
+// that several cells' words can be loaded together: occ_cell places the point
+// and reads its 8^3 block's coarse bit, occ_index names the cell in its
+// cascade's bitfield (asked only where the coarse bit is set: word index >> 6,
+// bit index & 63), and occ_skip stores the skip interval of the largest empty
+// box around an empty cell in sk (left unchanged outside every cascade).
+struct OccCell {
+  int ix, iy, iz, mip;  // mip >= nlvl: outside every cascade
+  bool block;           // its 8^3 block holds an occupied cell
+};
+FVC_HD OccCell occ_cell(V3 p, const OccParams& o, const uint32_t* coarse) {
   const V3 u = occ_unit(p, o);
   const float ax = fabsf(u.x - 0.5f), ay = fabsf(u.y - 0.5f), az = fabsf(u.z - 0.5f);
   const float mx = fmaxf(fmaxf(ax, ay), az);
   int e;
   frexpf(mx, &e);
   const int mip = e + 1 > 0 ? e + 1 : 0;
-  if (mip >= o.nlvl) return false;
+  if (mip >= o.nlvl) return OccCell{0, 0, 0, mip, false};
   const float scm = ldexpf(1.0f, -mip);
   const float px = (u.x - 0.5f) * scm + 0.5f, py = (u.y - 0.5f) * scm + 0.5f, pz = (u.z - 0.5f) * scm + 0.5f;
   int ix = (int)(px * 128.0f), iy = (int)(py * 128.0f), iz = (int)(pz * 128.0f);
@@ -166,14 +172,22 @@ FVC_HD bool occ_query(V3 p, const OccParams& o, const uint64_t* __restrict__ bf6
   iz = iz < 0 ? 0 : (iz > 127 ? 127 : iz);
   const uint32_t* cw = coarse + mip * COARSE_WORDS;
   const int b8 = (((ix >> 3) * 16) + (iy >> 3)) * 16 + (iz >> 3);
+  return OccCell{ix, iy, iz, mip, (bool)((cw[b8 >> 5] >> (b8 & 31)) & 1u)};
+}
+FVC_HD uint32_t occ_index(const OccCell& c) {
+  return morton3d((uint32_t)c.ix, (uint32_t)c.iy, (uint32_t)c.iz) + (uint32_t)c.mip * (CASCADE_WORDS64 * 64u);
+}
+// w: the cell's word (any value where block is not set)
+FVC_HD void occ_skip(const OccCell& c, uint64_t w, const OccParams& o, const uint32_t* coarse, const RaySlab& rs,
+                     Skip& sk) {
+  const int ix = c.ix, iy = c.iy, iz = c.iz, mip = c.mip;
+  if (mip >= o.nlvl) return;
   int g;
-  if ((cw[b8 >> 5] >> (b8 & 31)) & 1u) {
-    const uint32_t idx = morton3d((uint32_t)ix, (uint32_t)iy, (uint32_t)iz);
-    const uint64_t w = bf64[(idx >> 6) + (uint32_t)mip * CASCADE_WORDS64];
-    const uint32_t byte = (uint32_t)(w >> (idx & 56u)) & 0xffu;
-    if ((byte >> (idx & 7u)) & 1u) return true;
+  if (c.block) {
+    const uint32_t byte = (uint32_t)(w >> (occ_index(c) & 56u)) & 0xffu;
     g = w == 0 ? 4 : (byte == 0 ? 2 : 1);
   } else {
+    const uint32_t* cw = coarse + mip * COARSE_WORDS;
     const int b16 = (((ix >> 4) * 8) + (iy >> 4)) * 8 + (iz >> 4);
     const int b32 = (((ix >> 5) * 4) + (iy >> 5)) * 4 + (iz >> 5);
     const bool e16 = !((cw[COARSE8_WORDS + (b16 >> 5)] >> (b16 & 31)) & 1u);
@@ -181,6 +195,17 @@ FVC_HD bool occ_query(V3 p, const OccParams& o, const uint64_t* __restrict__ bf6
     g = e32 ? 32 : (e16 ? 16 : 8);
   }
   sk = box_skip(ix & -g, iy & -g, iz & -g, g, mip, o, rs);
+}
+FVC_HD bool occ_query(V3 p, const OccParams& o, const uint64_t* __restrict__ bf64, const uint32_t* coarse,
+                      const RaySlab& rs, Skip& sk) {
+  const OccCell c = occ_cell(p, o, coarse);
+  uint64_t w = 0;
+  if (c.block) {
+    const uint32_t i = occ_index(c);
+    w = bf64[i >> 6];
+    if ((w >> (i & 63u)) & 1u) return true;
+  }
+  occ_skip(c, w, o, coarse, rs, sk);
   return false;
 }
 

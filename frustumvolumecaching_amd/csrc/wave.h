@@ -21,15 +21,18 @@ __device__ __forceinline__ int wave_excl_scan(int v, int& total) {
   return x - v;
 }
 
-// Reserve `v` consecutive slots of *counter per lane (one atomic per wave);
-// returns this lane's first slot.  Every lane of the wave must call it.
-__device__ __forceinline__ int wave_reserve(int v, int* counter) {
-  int total;
-  const int prefix = wave_excl_scan(v, total);
-  int base = 0;
-  if (lane_id() == 0 && total > 0) base = atomicAdd(counter, total);
-  base = __shfl(base, 0, 64);
-  return base + prefix;
+// The same for 0 <= v < 2^BITS by ballots (no LDS round trips).
+template <int BITS>
+__device__ __forceinline__ int wave_excl_scan_bits(int v, int& total) {
+  int pre = 0;
+  total = 0;
+#pragma unroll
+  for (int b = 0; b < BITS; b++) {
+    const uint64_t m = __ballot((v >> b) & 1);
+    pre += (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0)) << b;
+    total += __popcll(m) << b;
+  }
+  return pre;
 }
 
 // Reserve v[c] consecutive slots of *ctr[c] per thread, for each of the N
