@@ -436,7 +436,7 @@ struct Renderer {
   std::vector<SceneRef> scene_refs_host;
   // fill scratch (own counters and pinned mirror: the fill may run on the
   // fill stream from another thread)
-  DevBuf f_rays, f_tiles, f_list, f_pos, f_t0, f_meta, f_out16, f_counters;
+  DevBuf f_rays, f_ray_t, f_state, f_tiles, f_list, f_pos, f_out16, f_counters;
   DevBuf f_bins;  // fill: start and midpoint of every bin of the frustum
   DevBuf f_alive8, f_alloc8;  // fill: alive byte per tile, brick-request byte per list entry
   DevBuf f_lsig;              // fill: log sigma per sample (half), plain models
