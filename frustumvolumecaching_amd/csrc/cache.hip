@@ -1528,13 +1528,22 @@ __global__ __launch_bounds__(256) void k_cache_composite(
     int kr = 0, kc = 0;
     int n_done = 0;       // samples composited
     // the two streams interleaved in march (= t0) order, batch by batch
-    for (int k0 = 0; group && k0 < n && visible; k0 += G) {
-      const int k = min(k0 + sub, n - 1);
+    uint2 v_next = make_uint2(0u, 0u);
+    float t_next = 0.0f;
+    auto load = [&](int at) {
+      const int k = min(at, n - 1);
       const int before = __popcll(ord & ((1ull << k) - 1ull));  // cache samples before sample k
       const bool from_cache = (ord >> k) & 1ull;
       const int q = from_cache ? e.z + before : e.x + k - before;
-      const uint2 v = (from_cache ? c_out : s_out)[q];
-      const float t = (from_cache ? c_t0 : s_t0)[q];
+      v_next = (from_cache ? c_out : s_out)[q];
+      t_next = (from_cache ? c_t0 : s_t0)[q];
+    };
+    if (group && n > 0) load(sub);
+    for (int k0 = 0; group && k0 < n && visible; k0 += G) {
+      // the next samples are loaded while these are composited
+      const uint2 v = v_next;
+      const float t = t_next;
+      load(k0 + G + sub);
       visible = G == 16 ? composite_group<16>(res, v, t, n - k0, st, alpha_thre, n_done)
                         : composite_group<4>(res, v, t, n - k0, st, alpha_thre, n_done);
     }

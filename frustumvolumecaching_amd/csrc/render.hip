@@ -205,10 +205,16 @@ __global__ __launch_bounds__(256) void k_composite(int* __restrict__ ctl, int pa
     bool visible = true;  // transmittance still above the early-stop threshold
     if (group) {
       int n_done = 0;
+      // the next samples are loaded while these are composited
+      auto at = [&](int k) { return e.x + min(k, max(e.y - 1, 0)); };
+      uint2 v_next = make_uint2(0u, 0u);
+      float t_next = 0.0f;
+      if (e.y > 0) { v_next = s_out[at(sub)]; t_next = s_t0[at(sub)]; }
       for (int k0 = 0; k0 < e.y && visible; k0 += G) {
-        const int q = e.x + min(k0 + sub, e.y - 1);
-        const uint2 v = s_out[q];
-        const float t = s_t0[q];
+        const uint2 v = v_next;
+        const float t = t_next;
+        v_next = s_out[at(k0 + G + sub)];
+        t_next = s_t0[at(k0 + G + sub)];
         visible = G == 16 ? composite_group<16>(res, v, t, e.y - k0, st, alpha_thre, n_done)
                           : composite_group<4>(res, v, t, e.y - k0, st, alpha_thre, n_done);
       }

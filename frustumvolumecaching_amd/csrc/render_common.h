@@ -225,27 +225,56 @@ __device__ __forceinline__ bool composite_sample(float4& res, uint2 v, float t0,
   if (!(alpha > alpha_thre)) return !(res.w < 1e-4f);
   return composite_add(res, alpha, composite_colour(v), alpha_thre);
 }
-// Up to G samples by a lane group, lane k holding sample k (n of them):
-// opacities and colours in parallel, then every lane runs the sequential
-// products of composite_add in order, so res is the same on all of them and
-// the same as one lane's.  Returns whether the ray stays visible; n_done
-// counts the samples composited.
+// Compositing of up to G samples by a lane group, lane k holding sample k.
+// The lanes form opacities, colours and weights in parallel; what a lane by
+// itself adds and multiplies one after the other stays in that order, on every
+// lane of the group, so results are the same bit for bit.
+// group_transmittance: T after all G samples, from each lane's factor
+// (1 - alpha, or 1 for a sample that does not count); returns T before the
+// lane's own.  group_add: acc + x of lane 0 + x of lane 1 ...
+// Measured with the broadcasts by LDS permutes (4 a sample) and each sample's
+// weight formed on every lane, then so, the next samples loaded ahead: a
+// launch of the full composite of 256x256 10.5 -> 8.3 us, of the reprojected
+// one of 640x360 25.0 -> 20.8 us; whole frames 1640 -> 1575 and 1160 -> 1150.
+template <int G>
+__device__ __forceinline__ float group_transmittance(float factor, float& T) {
+  const int sub = lane_id() & (G - 1);
+  float before = T;
+  each<G>([&](auto u) {
+    before = sub == u ? T : before;
+    T = T * group_lane<G, u>(factor);
+  });
+  return before;
+}
+template <int G>
+__device__ __forceinline__ float group_add(float acc, float x) {
+  each<G>([&](auto u) { acc = acc + group_lane<G, u>(x); });
+  return acc;
+}
+// Up to G samples of a ray, n of them in the stream: returns whether the ray
+// stays visible; n_done counts the samples composited.
 template <int G>
 __device__ __forceinline__ bool composite_group(float4& res, uint2 v, float t0, int n, const fvc_stepsize_info& st,
                                                 float alpha_thre, int& n_done) {
+  const int lane = lane_id(), sub = lane & (G - 1);
   const float alpha = composite_alpha(v, t0, st);
+  const bool counts = sub < n && alpha > alpha_thre;
+  const float factor = counts ? 1.0f - alpha : 1.0f;
+  float T = res.w;
+  const float before = group_transmittance<G>(factor, T);
+  const float after = before * factor;
+  // the sample that ends the ray, if any: those after it do not count
+  const uint32_t ends = (uint32_t)(__ballot(sub < n && after < 1e-4f) >> (lane & ~(G - 1))) & ((1u << G) - 1u);
+  const int last = ends ? __ffs(ends) - 1 : G - 1;
   const V3 c = composite_colour(v);
-  bool visible = true;
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    const float au = __shfl(alpha, u, G);
-    const V3 cu = V3{__shfl(c.x, u, G), __shfl(c.y, u, G), __shfl(c.z, u, G)};
-    if (u < n && visible) {
-      visible = composite_add(res, au, cu, alpha_thre);
-      n_done++;
-    }
-  }
-  return visible;
+  const bool adds = counts && sub <= last;
+  const float w = alpha * before;
+  res.x = group_add<G>(res.x, adds ? w * c.x : 0.0f);
+  res.y = group_add<G>(res.y, adds ? w * c.y : 0.0f);
+  res.z = group_add<G>(res.z, adds ? w * c.z : 0.0f);
+  res.w = ends ? __shfl(after, last, G) : T;
+  n_done += min(n, last + 1);
+  return ends == 0;
 }
 // to_8bit (raymarch_common.h:554-557)
 FVC_HD int to_8bit(float f) {

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 namespace fvc {
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
@@ -96,6 +98,26 @@ __device__ __forceinline__ int wave_min(int v) {
     v = o < v ? o : v;
   }
   return v;
+}
+
+// f(0), ..., f(N - 1) with compile-time arguments
+template <class F, int... U>
+__device__ __forceinline__ void each_impl(F&& f, std::integer_sequence<int, U...>) {
+  (f(std::integral_constant<int, U>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void each(F&& f) {
+  each_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// Value of lane U of the caller's group of G lanes (DPP: row_newbcast,
+// quad_perm), an operand modifier or one instruction and no LDS round trip.
+// The group's lanes must be active together.
+template <int G, int U>
+__device__ __forceinline__ float group_lane(float v) {
+  static_assert((G == 16 || G == 4) && U < G, "groups of 16 or 4 lanes");
+  const int b = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, b, G == 16 ? 0x150 + U : U * 0x55, 0xf, 0xf, false));
 }
 
 // LDS written by lanes of a wave, read by other lanes of the same wave
