@@ -887,7 +887,7 @@ void cache_fill(Renderer& r, const fvc_raymarch_info& rm, fvc_init_stats* stats,
 // of the ray in march order (0 skip, 1 resample, 2 cache), the first dbg_k
 // at dbg_codes[pixel * dbg_k ..], dbg_n[pixel] counting them across launches.
 static constexpr int CLS_EMIT = 16;  // samples whose t0 the emission loads together
-__global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int par, int trip_cutoff, MarchGrid mg,
+__global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ lg, StepPlan plan, int trip_cutoff, MarchGrid mg,
                                                      ContractParams con, const uint32_t* __restrict__ coarse_g,
                                                      CacheView cv, RayDyn* __restrict__ rays, int4* __restrict__ entry,
                                                      int* __restrict__ alive_flag, float* __restrict__ t_scr,
@@ -899,15 +899,16 @@ __global__ __launch_bounds__(256) void k_cache_march(int* __restrict__ ctl, int 
                                                      const RayState* __restrict__ rconst, int render_mode,
                                                      int8_t* __restrict__ dbg_codes, int dbg_k,
                                                      int* __restrict__ dbg_n) {
-  const int n_alive = ctl[CTL_ALIVE + par];
+  const int n_alive = lg[LOG_ALIVE];
   const int G = mg.tab.n_rows > 0 ? group_lanes(n_alive) : 1;
   const bool group = G > 1;
   const int rays_per_block = 256 / G;
   if ((int)blockIdx.x * rays_per_block >= n_alive) return;  // whole block past the alive rays
-  const int n_steps = ctl[CTL_NSTEPS];
-  int* cnt_r = ctl + CTL_R;
-  int* cnt_c = ctl + CTL_C;
-  int* step_counter = ctl + CTL_BINS;
+  const int n_steps = plan_steps(plan, n_alive);
+  if (blockIdx.x == 0 && threadIdx.x == 0) lg[LOG_STEPS] = n_steps;
+  int* cnt_r = lg + LOG_R;
+  int* cnt_c = lg + LOG_C;
+  int* step_counter = lg + LOG_BINS;
   extern __shared__ uint32_t coarse[];  // march_lds
   load_coarse(coarse_g, mg.occ.nlvl, coarse);
   const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
@@ -1496,7 +1497,7 @@ __global__ __launch_bounds__(256) void k_cache_head_vd(const float4* __restrict_
 // the resample and cache streams of a ray by t0 (resample first iff t0_r <
 // t0_c) and composite; then compact the alive rays.
 __global__ __launch_bounds__(256) void k_cache_composite(
-    int* __restrict__ ctl, int par, fvc_stepsize_info st, float alpha_thre, const RayDyn* __restrict__ rays_in,
+    int* __restrict__ lg, fvc_stepsize_info st, float alpha_thre, const RayDyn* __restrict__ rays_in,
     const int* __restrict__ pix_in, const float4* __restrict__ res_in, const int4* __restrict__ entry,
     const uint64_t* __restrict__ order, const int* __restrict__ alive_flag, const uint2* __restrict__ s_out,
     const float* __restrict__ s_t0, const uint2* __restrict__ c_out, const float* __restrict__ c_t0,
@@ -1504,12 +1505,12 @@ __global__ __launch_bounds__(256) void k_cache_composite(
     float4* __restrict__ results, int2* __restrict__ dbg_comp) {
   // dbg_comp (optional, inspection only): per pixel the resampled and cached
   // samples composited, up to and including the one that ends the ray
-  const int n_alive = ctl[CTL_ALIVE + par];
+  const int n_alive = lg[LOG_ALIVE];
   const int G = group_lanes(n_alive);
   const bool group = G > 1;
   const int rays_per_block = 256 / G;
   if ((int)blockIdx.x * rays_per_block >= n_alive) return;
-  int* counter = ctl + CTL_ALIVE + (par ^ 1);
+  int* counter = lg + CTL_LOG_FIELDS + LOG_ALIVE;  // the next iteration's
   const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
   const int sub = threadIdx.x & (G - 1);
   const bool valid = i < n_alive;
@@ -1618,6 +1619,7 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
   int* ctl = r.counters.as<int>();
   const int64_t target = std::min<int64_t>(vs.target(r.target_batch), cap - 64);
   const int64_t n_bound = std::min<int64_t>(cap - 64, (int64_t)n0 * r.max_steps);  // samples per launch
+  const StepPlan plan = step_plan(target, r.max_steps, cap - 64);
   const dim3 grid(ray_blocks(n0));
   const int head_blocks = (int)std::min<int64_t>((n_bound + 255) / 256, 256 * 16);
   // loop trips per ray and launch; a performance knob only (a ray resumes
@@ -1628,10 +1630,9 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
   std::vector<Handles> hs;
   auto iteration = [&](int it) {
       const int cur = it & 1;
-      hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, target, r.max_steps, cap - 64, 0);
       Handles h;
       ev = P.begin(s);
-      hipLaunchKernelGGL(k_cache_march, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl, cur, cutoff, mg, m.con, m.coarse.as<uint32_t>(), cv,
+      hipLaunchKernelGGL(k_cache_march, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl + ctl_at(it, 0), plan, cutoff, mg, m.con, m.coarse.as<uint32_t>(), cv,
                          r.rays[cur].as<RayDyn>(), r.ray_entry.as<int4>(), r.ray_alive.as<int>(),
                          r.t_scratch.as<float>(), r.s_pos.as<float4>(), r.s_t0.as<float>(), r.c_rec.as<float4>(), r.c_t0.as<float>(), r.ray_pix[cur].as<int>(), r.ray_sh.as<uint4>(),
                          m.net.split_head ? r.ray_od.as<float4>() : nullptr,
@@ -1641,13 +1642,13 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       h.march = P.end(ev, s, "cache_march");
       ev = P.begin(s);
       launch_network_full_pix(m, r.s_pos.as<float4>(), r.ray_sh.as<uint4>(), n_bound, r.s_out.as<uint32_t>(), s,
-                              ctl + CTL_R, r.mlp_rows, false);
+                              ctl + ctl_at(it, LOG_R), r.mlp_rows, false);
       h.net = P.end(ev, s, "network_resample");
       ev = P.begin(s);
 #define L2(P, F8)                                                                                                    \
   hipLaunchKernelGGL((k_cache_head<P, F8>), dim3(head_blocks), dim3(256), 0, s, r.c_rec.as<float4>(),                 \
                      r.ray_sh.as<uint4>(), (int64_t)n_bound, cv, m.frags.as<typename Mx<P>::T>(), m.mlp_scales,       \
-                     di_plain, r.c_out.as<uint2>(), ctl + CTL_C)
+                     di_plain, r.c_out.as<uint2>(), ctl + ctl_at(it, LOG_C))
 #define L(P)                     \
   if (cv.lat8) { L2(P, true); }  \
   else { L2(P, false); }
@@ -1655,7 +1656,7 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
         hipLaunchKernelGGL(k_cache_head_vd, dim3(head_blocks), dim3(256), 0, s, r.c_rec.as<float4>(),
                            r.c_t0.as<float>(), r.ray_sh.as<uint4>(), r.ray_od.as<float4>(), (int64_t)n_bound, cv,
                            rm.stepsize_info, m.con, m.frags.as<h8>(), m.net.first_latent_is_density,
-                           m.net.freq_encoding_degree > 0, r.c_out.as<uint2>(), ctl + CTL_C);
+                           m.net.freq_encoding_degree > 0, r.c_out.as<uint2>(), ctl + ctl_at(it, LOG_C));
       } else {
         switch (m.net.precision) {
           case FVC_PREC_BF16: L(FVC_PREC_BF16); break;
@@ -1669,7 +1670,7 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       FVC_HIP(hipGetLastError());
       h.head = P.end(ev, s, "cache_head");
       ev = P.begin(s);
-      hipLaunchKernelGGL(k_cache_composite, grid, dim3(256), 0, s, ctl, cur, rm.stepsize_info, m.scene.alpha_thre,
+      hipLaunchKernelGGL(k_cache_composite, grid, dim3(256), 0, s, ctl + ctl_at(it, 0), rm.stepsize_info, m.scene.alpha_thre,
                          r.rays[cur].as<RayDyn>(), r.ray_pix[cur].as<int>(), r.ray_res[cur].as<float4>(),
                          r.ray_entry.as<int4>(), r.ray_order.as<uint64_t>(), r.ray_alive.as<int>(),
                          r.s_out.as<uint2>(), r.s_t0.as<float>(), r.c_out.as<uint2>(), r.c_t0.as<float>(),
@@ -1688,14 +1689,13 @@ void render_cached(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       for (int i = 0; i < k; i++) iteration(i);
     });
     it = k;
-    done = read_counter(r, CTL_ALIVE + (it & 1), s) == 0;
+    done = read_counter(r, ctl_at(it, LOG_ALIVE), s) == 0;
   }
   while (!done && it < MAX_SUBITER) {
     const int burst = next_burst(r, it);
     for (int b = 0; b < burst && it < MAX_SUBITER; b++, it++) iteration(it);
-    done = read_counter(r, CTL_ALIVE + (it & 1), s) == 0;
+    done = read_counter(r, ctl_at(it, LOG_ALIVE), s) == 0;
   }
-  hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, target, r.max_steps, cap - 64, 1);
   ev = P.begin(s);
   launch_write_image(r, vs, s);
   P.end(ev, s, "write_image", n_px, n_px * 24, 0);

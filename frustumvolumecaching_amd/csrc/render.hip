@@ -66,21 +66,22 @@ static constexpr int EMIT = 16;  // samples whose t0 the full marcher's emission
 // scene (scenes[scene]) with the coarse table from global memory (L2
 // resident) instead of the block's LDS copy.
 template <bool MULTI>
-__global__ __launch_bounds__(256) void k_march(int* __restrict__ ctl, int par, MarchGrid mg, ContractParams con,
+__global__ __launch_bounds__(256) void k_march(int* __restrict__ lg, StepPlan plan, MarchGrid mg, ContractParams con,
                                                const uint32_t* __restrict__ coarse_g,
                                                const SceneRef* __restrict__ scenes, RayDyn* __restrict__ rays,
                                                const RayState* __restrict__ rconst, const int* __restrict__ pix_in,
                                                int4* __restrict__ entry, int* __restrict__ alive_flag,
                                                float* __restrict__ t_scr, float4* __restrict__ s_pos,
                                                uint4* __restrict__ ray_sh, float* __restrict__ s_t0) {
-  const int n_alive = ctl[CTL_ALIVE + par];
+  const int n_alive = lg[LOG_ALIVE];
   const int G = mg.tab.n_rows > 0 ? group_lanes(n_alive) : 1;
   const bool group = G > 1;
   const int rays_per_block = 256 / G;
   if ((int)blockIdx.x * rays_per_block >= n_alive) return;  // whole block past the alive rays
-  const int n_steps = ctl[CTL_NSTEPS];
-  int* s_counter = ctl + CTL_R;
-  int* step_counter = ctl + CTL_BINS;
+  const int n_steps = plan_steps(plan, n_alive);
+  if (blockIdx.x == 0 && threadIdx.x == 0) lg[LOG_STEPS] = n_steps;
+  int* s_counter = lg + LOG_R;
+  int* step_counter = lg + LOG_BINS;
   extern __shared__ uint32_t coarse[];  // march_lds
   if constexpr (!MULTI) load_coarse(coarse_g, mg.occ.nlvl, coarse);
   const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
@@ -177,19 +178,19 @@ __global__ __launch_bounds__(256) void k_march(int* __restrict__ ctl, int par, M
 // compaction of the next sub-iteration (renderer.cu:158-189).  The samples
 // of a ray are read in batches of COMPOSITE_BATCH independent loads ahead of
 // the sequential compositing.
-__global__ __launch_bounds__(256) void k_composite(int* __restrict__ ctl, int par, fvc_stepsize_info st,
+__global__ __launch_bounds__(256) void k_composite(int* __restrict__ lg, fvc_stepsize_info st,
                                                    float alpha_thre, const RayDyn* __restrict__ rays_in,
                                                    const int* __restrict__ pix_in, const float4* __restrict__ res_in,
                                                    const int4* __restrict__ entry, const int* __restrict__ alive_flag,
                                                    const uint2* __restrict__ s_out, const float* __restrict__ s_t0,
                                                    RayDyn* __restrict__ rays_out, int* __restrict__ pix_out,
                                                    float4* __restrict__ res_out, float4* __restrict__ results) {
-  const int n_alive = ctl[CTL_ALIVE + par];
+  const int n_alive = lg[LOG_ALIVE];
   const int G = group_lanes(n_alive);
   const bool group = G > 1;
   const int rays_per_block = 256 / G;
   if ((int)blockIdx.x * rays_per_block >= n_alive) return;
-  int* counter = ctl + CTL_ALIVE + (par ^ 1);
+  int* counter = lg + CTL_LOG_FIELDS + LOG_ALIVE;  // the next iteration's
   const int i = blockIdx.x * rays_per_block + threadIdx.x / G;
   const int sub = threadIdx.x & (G - 1);
   const bool valid = i < n_alive;
@@ -326,28 +327,6 @@ void ensure_ray_capacity(Renderer& r, int64_t n, int64_t target) {
   if (!r.pinned) FVC_HIP(hipHostMalloc((void**)&r.pinned, 64 * sizeof(int), hipHostMallocDefault));
 }
 
-__global__ void k_plan(int* __restrict__ ctl, int it, int64_t target, int max_steps, int64_t cap, int log_only) {
-  if (threadIdx.x != 0) return;
-  if (it > 0 && it - 1 <= MAX_SUBITER) {
-    int* lg = ctl + CTL_LOG + CTL_LOG_FIELDS * (it - 1);
-    lg[0] = ctl[CTL_ALIVE + ((it - 1) & 1)];
-    lg[1] = ctl[CTL_NSTEPS];
-    lg[2] = ctl[CTL_R];
-    lg[3] = ctl[CTL_C];
-    lg[4] = ctl[CTL_BINS];
-  }
-  if (log_only) return;
-  const int64_t n = ctl[CTL_ALIVE + (it & 1)];
-  int64_t k = target / (n > 1 ? n : 1);
-  k = k < 1 ? 1 : (k > max_steps ? max_steps : k);
-  if (n > 0 && n * k > cap) k = cap / n > 1 ? cap / n : 1;
-  ctl[CTL_NSTEPS] = (int)k;
-  ctl[CTL_R] = 0;
-  ctl[CTL_C] = 0;
-  ctl[CTL_BINS] = 0;
-  ctl[CTL_ALIVE + ((it + 1) & 1)] = 0;
-}
-
 std::vector<IterLog> read_iter_log(Renderer& r, int n_it, hipStream_t s) {
   std::vector<IterLog> out((size_t)n_it);
   if (n_it > 0) {
@@ -359,9 +338,9 @@ std::vector<IterLog> read_iter_log(Renderer& r, int n_it, hipStream_t s) {
 }
 
 int read_counter(Renderer& r, int idx, hipStream_t s) {
-  FVC_HIP(hipMemcpyAsync(r.pinned + idx, r.counters.as<int>() + idx, sizeof(int), hipMemcpyDeviceToHost, s));
+  FVC_HIP(hipMemcpyAsync(r.pinned, r.counters.as<int>() + idx, sizeof(int), hipMemcpyDeviceToHost, s));
   FVC_HIP(hipStreamSynchronize(s));
-  return r.pinned[idx];
+  return r.pinned[0];
 }
 
 __global__ void k_zero_ints(int* __restrict__ p, int n) {
@@ -371,7 +350,7 @@ __global__ void k_zero_ints(int* __restrict__ p, int n) {
 
 // a kernel, not a memset: the frame may be recorded into a graph
 void zero_counters(Renderer& r, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(CTL_LOG), 0, s, r.counters.as<int>(), CTL_LOG);
+  hipLaunchKernelGGL(k_zero_ints, dim3((CTL_WORDS + 255) / 256), dim3(256), 0, s, r.counters.as<int>(), CTL_WORDS);
   FVC_HIP(hipGetLastError());
 }
 
@@ -449,7 +428,7 @@ Views::Views(const fvc_raymarch_info* rms_, int n_, uint8_t* const* rgba_, const
 // counter); returns the number of alive rays.
 int launch_init_rays(Renderer& r, const Views& vs, hipStream_t s) {
   launch_init_rays_async(r, vs, s);
-  return read_counter(r, CTL_ALIVE, s);
+  return read_counter(r, ctl_at(0, LOG_ALIVE), s);
 }
 
 void launch_init_rays_async(Renderer& r, const Views& vs, hipStream_t s) {
@@ -461,7 +440,7 @@ void launch_init_rays_async(Renderer& r, const Views& vs, hipStream_t s) {
     hipLaunchKernelGGL(k_init_rays, dim3((W + 31) / 32, (H + 31) / 32), dim3(INIT_BLOCK), 0, s, rm, (int)vs.base[v],
                        vs.scene[v], cvt(m.scene.aabb_from), cvt(m.scene.aabb_to), r.rays[0].as<RayDyn>(),
                        r.ray_const.as<RayState>(), r.ray_pix[0].as<int>(), r.ray_res[0].as<float4>(),
-                       r.results.as<float4>(), r.counters.as<int>() + CTL_ALIVE);
+                       r.results.as<float4>(), r.counters.as<int>() + ctl_at(0, LOG_ALIVE));
     FVC_HIP(hipGetLastError());
   }
 }
@@ -552,15 +531,8 @@ void upload_scene_refs(Renderer& r, const Views& vs) {
   r.scene_refs_host = refs;
 }
 
-int steps_for(int n_alive, int64_t target, int max_steps) {
-  int64_t k = target / std::max(n_alive, 1);
-  if (k < 1) k = 1;
-  if (k > max_steps) k = max_steps;
-  return (int)k;
-}
-
 // Sub-iterations are launched in bursts with their counts kept on the
-// device (k_plan); the host reads the alive count once per burst.  The
+// device; the host reads the alive count once per burst.  The
 // first burst is as long as the previous frame's loop.
 int next_burst(const Renderer& r, int it) { return it == 0 ? std::max(2, r.last_iters) : 2; }
 
@@ -585,15 +557,15 @@ void render_full(Renderer& r, const Views& vs, fvc_render_stats* stats) {
   const int64_t cap = r.sample_capacity - 64;
   const int64_t target = std::min<int64_t>(vs.target(r.target_batch), cap);
   const int64_t n_bound = std::min<int64_t>(cap, (int64_t)n0 * r.max_steps);  // samples per launch
+  const StepPlan plan = step_plan(target, r.max_steps, cap);
   const dim3 grid(ray_blocks(n0));
   struct Handles { int march, net, comp; };
   std::vector<Handles> hs;
   auto iteration = [&](int it) {
       const int cur = it & 1;
-      hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, target, r.max_steps, cap, 0);
       Handles h;
       ev = P.begin(s);
-      hipLaunchKernelGGL(multi ? k_march<true> : k_march<false>, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl, cur, mg, m.con,
+      hipLaunchKernelGGL(multi ? k_march<true> : k_march<false>, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl + ctl_at(it, 0), plan, mg, m.con,
                          m.coarse.as<uint32_t>(), r.scene_refs.as<SceneRef>(), r.rays[cur].as<RayDyn>(), r.ray_const.as<RayState>(), r.ray_pix[cur].as<int>(),
                          r.ray_entry.as<int4>(), r.ray_alive.as<int>(), r.t_scratch.as<float>(),
                          r.s_pos.as<float4>(), r.ray_sh.as<uint4>(), r.s_t0.as<float>());
@@ -601,10 +573,10 @@ void render_full(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       h.march = P.end(ev, s, "march");
       ev = P.begin(s);
       launch_network_full_pix(m, r.s_pos.as<float4>(), r.ray_sh.as<uint4>(), n_bound, r.s_out.as<uint32_t>(), s,
-                              ctl + CTL_R, r.mlp_rows, true);
+                              ctl + ctl_at(it, LOG_R), r.mlp_rows, true);
       h.net = P.end(ev, s, "network_full");
       ev = P.begin(s);
-      hipLaunchKernelGGL(k_composite, grid, dim3(256), 0, s, ctl, cur, rm.stepsize_info, m.scene.alpha_thre,
+      hipLaunchKernelGGL(k_composite, grid, dim3(256), 0, s, ctl + ctl_at(it, 0), rm.stepsize_info, m.scene.alpha_thre,
                          r.rays[cur].as<RayDyn>(), r.ray_pix[cur].as<int>(), r.ray_res[cur].as<float4>(),
                          r.ray_entry.as<int4>(), r.ray_alive.as<int>(), r.s_out.as<uint2>(), r.s_t0.as<float>(),
                          r.rays[cur ^ 1].as<RayDyn>(), r.ray_pix[cur ^ 1].as<int>(),
@@ -622,14 +594,13 @@ void render_full(Renderer& r, const Views& vs, fvc_render_stats* stats) {
       for (int i = 0; i < k; i++) iteration(i);
     });
     it = k;
-    done = read_counter(r, CTL_ALIVE + (it & 1), s) == 0;
+    done = read_counter(r, ctl_at(it, LOG_ALIVE), s) == 0;
   }
   while (!done && it < MAX_SUBITER) {
     const int burst = next_burst(r, it);
     for (int b = 0; b < burst && it < MAX_SUBITER; b++, it++) iteration(it);
-    done = read_counter(r, CTL_ALIVE + (it & 1), s) == 0;
+    done = read_counter(r, ctl_at(it, LOG_ALIVE), s) == 0;
   }
-  hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, target, r.max_steps, cap, 1);
   ev = P.begin(s);
   launch_write_image(r, vs, s);
   P.end(ev, s, "write_image", n_px, n_px * 24, 0);
@@ -751,23 +722,23 @@ void render_full_noalloc(Renderer& r, const fvc_raymarch_info& rm, uint8_t* rgba
   mg.tab.n_rows = 0;
   mg.bf64 = m.bitfield.as<uint64_t>();
 
-  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(CTL_LOG), 0, s, ctl, CTL_LOG);
+  hipLaunchKernelGGL(k_zero_ints, dim3((CTL_WORDS + 255) / 256), dim3(256), 0, s, ctl, CTL_WORDS);
   hipLaunchKernelGGL(k_init_rays, dim3((W + 31) / 32, (H + 31) / 32), dim3(INIT_BLOCK), 0, s, rm, 0, 0,
-                     cvt(m.scene.aabb_from), cvt(m.scene.aabb_to), rays[0], rconst, pix[0], rres[0], results, ctl + CTL_ALIVE);
+                     cvt(m.scene.aabb_from), cvt(m.scene.aabb_to), rays[0], rconst, pix[0], rres[0], results, ctl + ctl_at(0, LOG_ALIVE));
   FVC_HIP(hipGetLastError());
   const int64_t cap = S - 64;
   const int64_t n_bound = std::min<int64_t>(cap, P * NOALLOC_STEPS);
+  const StepPlan plan = step_plan(cap, NOALLOC_STEPS, cap);
   const dim3 grid(ray_blocks(P));
   auto iteration = [&](int it) {
     const int cur = it & 1;
-    hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, cap, NOALLOC_STEPS, cap, 0);
-    hipLaunchKernelGGL(k_march<false>, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl, cur, mg, m.con, m.coarse.as<uint32_t>(), nullptr,
+    hipLaunchKernelGGL(k_march<false>, grid, dim3(256), march_lds(mg.occ.nlvl), s, ctl + ctl_at(it, 0), plan, mg, m.con, m.coarse.as<uint32_t>(), nullptr,
                        rays[cur], rconst,
                        pix[cur], entry, alive, t_scr, s_pos, ray_sh, s_t0);
     FVC_HIP(hipGetLastError());
-    launch_network_full_pix(m, s_pos, ray_sh, n_bound, reinterpret_cast<uint32_t*>(s_out), s, ctl + CTL_R,
-                            r.mlp_rows, false);
-    hipLaunchKernelGGL(k_composite, grid, dim3(256), 0, s, ctl, cur, rm.stepsize_info, m.scene.alpha_thre, rays[cur],
+    launch_network_full_pix(m, s_pos, ray_sh, n_bound, reinterpret_cast<uint32_t*>(s_out), s,
+                            ctl + ctl_at(it, LOG_R), r.mlp_rows, false);
+    hipLaunchKernelGGL(k_composite, grid, dim3(256), 0, s, ctl + ctl_at(it, 0), rm.stepsize_info, m.scene.alpha_thre, rays[cur],
                        pix[cur], rres[cur], entry, alive, s_out, s_t0, rays[cur ^ 1], pix[cur ^ 1], rres[cur ^ 1],
                        results);
     FVC_HIP(hipGetLastError());
@@ -781,11 +752,10 @@ void render_full_noalloc(Renderer& r, const fvc_raymarch_info& rm, uint8_t* rgba
       throw Error(FVC_E_INVALID, "the no-allocation render needs more than 256 sub-iterations for this view");
     for (int b = 0; b < 4 && it < NOALLOC_MAX_ITERS; b++, it++) iteration(it);
     int n_alive = 0;
-    FVC_HIP(hipMemcpyAsync(&n_alive, ctl + CTL_ALIVE + (it & 1), sizeof(int), hipMemcpyDeviceToHost, s));
+    FVC_HIP(hipMemcpyAsync(&n_alive, ctl + ctl_at(it, LOG_ALIVE), sizeof(int), hipMemcpyDeviceToHost, s));
     FVC_HIP(hipStreamSynchronize(s));
     done = n_alive == 0;
   }
-  hipLaunchKernelGGL(k_plan, dim3(1), dim3(64), 0, s, ctl, it, cap, NOALLOC_STEPS, cap, 1);
   if (rgba) {
     hipLaunchKernelGGL(k_write_image, dim3((W + 15) / 16, (H + 15) / 16), dim3(256), 0, s, W, H, 0, results,
                        (uchar4*)rgba, rm.sample_index);

@@ -68,19 +68,34 @@ enum { CNT_ALIVE = 0, CNT_SAMPLES = 1, CNT_CACHE = 2, CNT_STEPS = 3, CNT_TILES =
        CNT_UNORDERED = 7, CNT_SLOTS = 8 /* and 9 */ };
 
 // Device control block of a frame's sub-iteration loop (also in
-// Renderer::counters): alive counts (ping-pong by iteration parity), the
-// samples per ray of the current iteration, the stream and bin counters,
-// and a per-iteration log {alive, n_steps, resample, cache, bins}.  The host
-// launches iterations in bursts and reads the alive count once per burst.
-enum { CTL_ALIVE = 16, CTL_NSTEPS = 18, CTL_R = 19, CTL_C = 20, CTL_BINS = 21, CTL_LOG = 32 };
+// Renderer::counters): one record per iteration, all zero when the frame
+// starts.  Iteration it's marcher reads its alive count, plans the samples per
+// ray from it and counts the samples and bins; its composite counts the rays
+// left into the next record.  The host launches iterations in bursts, reads
+// the alive count once per burst and the records at the end.
+// (A kernel of its own that planned each iteration took 4 us and a launch gap:
+// 256x256 1580 -> 1533 us a frame, 1279x717 1355 -> 1330, 1920x1080 11735 ->
+// 11675.)
+enum { CTL_LOG = 32 };
+enum { LOG_ALIVE = 0, LOG_STEPS = 1, LOG_R = 2, LOG_C = 3, LOG_BINS = 4 };
 static const int CTL_LOG_FIELDS = 5;
 static const int MAX_SUBITER = 1000;        // PerformanceRenderer::MAX_SUBITER
 static const int CTL_WORDS = CTL_LOG + CTL_LOG_FIELDS * (MAX_SUBITER + 1);
+inline int ctl_at(int it, int field) { return CTL_LOG + CTL_LOG_FIELDS * it + field; }
 
-// Plan iteration it: log iteration it-1, set the samples per ray
-// (TARGET_BATCH_SIZE / n_alive clamped to [1, max_steps] and to the stream
-// capacity, performance_renderer.cu:249-250) and zero the counters.
-__global__ void k_plan(int* __restrict__ ctl, int it, int64_t target, int max_steps, int64_t cap, int log_only);
+// Samples per ray of an iteration: TARGET_BATCH_SIZE / n_alive clamped to
+// [1, max_steps] and to the stream capacity (performance_renderer.cu:249-250).
+struct StepPlan { int target, max_steps, cap; };
+inline StepPlan step_plan(int64_t target, int max_steps, int64_t cap) {
+  const int64_t top = 0x7fffffff;
+  return StepPlan{(int)std::min(target, top), max_steps, (int)std::min(cap, top)};
+}
+FVC_HD int plan_steps(const StepPlan& p, int n) {
+  int k = p.target / (n > 1 ? n : 1);
+  k = k < 1 ? 1 : (k > p.max_steps ? p.max_steps : k);
+  if (n > 0 && (int64_t)n * k > p.cap) k = p.cap / n > 1 ? p.cap / n : 1;
+  return k;
+}
 
 inline CacheView cache_view(const CacheStore& C) {
   CacheView cv;
@@ -295,7 +310,6 @@ void prepare_views(Renderer& r, const Views& vs);
 struct IterLog { int alive, n_steps, n_r, n_c, bins; };
 std::vector<IterLog> read_iter_log(Renderer& r, int n_it, hipStream_t s);
 void launch_write_image(Renderer& r, const Views& vs, hipStream_t s);
-int steps_for(int n_alive, int64_t target, int max_steps);
 int next_burst(const Renderer& r, int it);
 
 }  // namespace fvc
