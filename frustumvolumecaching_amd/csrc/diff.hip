@@ -1337,18 +1337,34 @@ static void scatter_table(DiffState& D, const GridParams& gp, const int* list, i
   LevelList ll{};
   BinLevels bl{};
   int n_bins = 0, most = 1;
-  for (int l = 0; l < gp.n_levels; l++) {
-    const GridLevel& L = gp.lv[l];
-    const int nb = (int)((L.size + BIN_ENTRIES - 1) / BIN_ENTRIES);
-    if (n < BIN_MIN_SAMPLES || ((gp.dense_mask >> l) & 1u) || nb > BIN_MAX || L.res >= (uint32_t)BIN_ENTRIES) {
-      ll.l[ll.n++] = l;
-      continue;
+  auto plan = [&](bool bins) {
+    ll = LevelList{};
+    bl = BinLevels{};
+    n_bins = 0;
+    for (int l = 0; l < gp.n_levels; l++) {
+      const GridLevel& L = gp.lv[l];
+      const int nb = (int)((L.size + BIN_ENTRIES - 1) / BIN_ENTRIES);
+      if (!bins || ((gp.dense_mask >> l) & 1u) || nb > BIN_MAX || L.res >= (uint32_t)BIN_ENTRIES) {
+        ll.l[ll.n++] = l;
+        continue;
+      }
+      bl.l[bl.n] = l;
+      bl.n_bins[bl.n] = nb;
+      bl.first[bl.n++] = n_bins;
+      n_bins += nb;
+      most = std::max(most, nb);
     }
-    bl.l[bl.n] = l;
-    bl.n_bins[bl.n] = nb;
-    bl.first[bl.n++] = n_bins;
-    n_bins += nb;
-    most = std::max(most, nb);
+  };
+  plan(n >= BIN_MIN_SAMPLES);
+  // room for a quarter more than an even spread of four records a sample
+  const int64_t chunk = std::min<int64_t>(n, BIN_CHUNK);
+  const int cap = (int)(5 * chunk / most + 1024);
+  if (bl.n > 0 && !(D.bin_cursor.try_ensure((size_t)n_bins * sizeof(int)) &&
+                    D.bin_val.try_ensure((size_t)n_bins * cap * sizeof(float4)) &&
+                    D.bin_key.try_ensure((size_t)n_bins * cap * sizeof(uint32_t)))) {
+    D.bin_val.release();  // no room for the records: by atomics
+    D.bin_key.release();
+    plan(false);
   }
   if (ll.n > 0) {
     const int64_t per_block = 4 * 16 * SCATTER_SEG;
@@ -1357,12 +1373,6 @@ static void scatter_table(DiffState& D, const GridParams& gp, const int* list, i
     FVC_HIP(hipGetLastError());
   }
   if (bl.n == 0) return;
-  // room for a quarter more than an even spread of four records a sample
-  const int64_t chunk = std::min<int64_t>(n, BIN_CHUNK);
-  const int cap = (int)(5 * chunk / most + 1024);
-  D.bin_cursor.ensure((size_t)n_bins * sizeof(int));
-  D.bin_val.ensure((size_t)n_bins * cap * sizeof(float4));
-  D.bin_key.ensure((size_t)n_bins * cap * sizeof(uint32_t));
   hipLaunchKernelGGL(k_diff_zero, dim3((n_bins + 255) / 256), dim3(256), 0, s, D.bin_cursor.as<int>(), n_bins);
   for (int64_t c0 = 0; c0 < n; c0 += chunk) {
     const int64_t nc = std::min<int64_t>(chunk, n - c0);
@@ -1497,8 +1507,10 @@ void diff_backward(Renderer& r, const float* d_rgb, float* g_pos, float* g_base,
                      D.ray_out.as<float4>(), d_rgb, D.d_out4.as<float4>());
   FVC_HIP(hipGetLastError());
   if (D.n_r > 0) {
-    // the encoding's gradients pass through memory in chunks (at most 512 MiB)
-    const int64_t cap = std::min<int64_t>(D.n_r, (int64_t)1 << 22);
+    // the encoding's gradients pass through memory in chunks (at most 512 MiB,
+    // less where the device has no room)
+    int64_t cap = std::min<int64_t>(D.n_r, (int64_t)1 << 22);
+    while (cap > 4096 && !D.d_enc.try_ensure((size_t)cap * 16 * sizeof(float2))) cap = (cap + 1) / 2;
     D.d_enc.ensure((size_t)cap * 16 * sizeof(float2));
     const int* list = D.cached ? D.list_r.as<int>() : nullptr;
     for (int64_t j0 = 0; j0 < D.n_r; j0 += cap) {

@@ -54,6 +54,20 @@ struct DevBuf {
     FVC_HIP(hipMalloc(&p, n));
     bytes = n;
   }
+  // the same for a workspace that a caller can do without (or with less of):
+  // false, and the buffer empty, where the device has no room
+  bool try_ensure(size_t n) {
+    try {
+      ensure(n);
+    } catch (const Error& e) {
+      if (e.code != FVC_E_OUT_OF_MEMORY) throw;
+      (void)hipGetLastError();
+      p = nullptr;
+      bytes = 0;
+      return false;
+    }
+    return true;
+  }
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
