@@ -313,12 +313,17 @@ inline StepTableView step_view(const fvc_stepsize_info& st) {
 // the bin midpoint passes lim.  Returns the number of rows, 0 when the
 // table would exceed 200000 rows or 64 Mi entries (the marchers then step
 // every bin).
+// (On the host; the renderer builds the same table on the device.)
+static const int64_t STEP_TABLE_MAX = (int64_t)64 << 20;
+inline int step_rows(const fvc_stepsize_info& st, float lim) {
+  const double rows_d = std::ceil((double)step_from_t(st, lim) - (double)st.near_i) + 2.0;
+  return rows_d > 0 && rows_d < 200000 ? (int)rows_d : 0;
+}
 inline int build_step_rows(const fvc_stepsize_info& st, float lim, std::vector<float>& t, std::vector<int>& off) {
   t.clear();
   off.clear();
-  const double rows_d = std::ceil((double)step_from_t(st, lim) - (double)st.near_i) + 2.0;
-  if (!(rows_d > 0 && rows_d < 200000)) return 0;
-  const int rows = (int)rows_d;
+  const int rows = step_rows(st, lim);
+  if (rows == 0) return 0;
   off.reserve(rows + 1);
   for (int m = 0; m < rows; m++) {
     off.push_back((int)t.size());
@@ -330,7 +335,7 @@ inline int build_step_rows(const fvc_stepsize_info& st, float lim, std::vector<f
       t.push_back(t1);
       if ((t0 + t1) * 0.5f > lim) break;
     }
-    if (t.size() > ((size_t)64 << 20)) {
+    if ((int64_t)t.size() > STEP_TABLE_MAX) {
       t.clear();
       off.clear();
       return 0;
