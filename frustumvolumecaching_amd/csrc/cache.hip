@@ -35,7 +35,6 @@ struct FillRay {
 static const int FILL_ALIVE = 256;
 struct FillState {
   int flags;  // FILL_ALIVE; bit j < 8: the ray has a sample in bin j of its tile's slab
-  int next;   // its first occupied bin from the tile's slab on (k_fill_sample); below that slab: not known
 };
 struct FillTile {
   int slab, alive, n_bricks, processed;
@@ -72,7 +71,7 @@ __global__ __launch_bounds__(64) void k_fill_init(fvc_raymarch_info rm, V3 aabb_
   const int64_t i = (int64_t)t * 64 + lane;
   rays[i] = FillRay{r.d.x, r.d.y, r.d.z, hit ? fminf_(a1, s.far_) : s.far_};
   ray_T[i] = 1.0f;
-  state[i] = FillState{hit ? FILL_ALIVE : 0, -1};
+  state[i] = FillState{hit ? FILL_ALIVE : 0};
   int start = (int)(step_from_t(s, hit ? a0 : s.near_) - s.near_i);
   start = start > 0 ? start : 0;
   const int mn = wave_min(start);
@@ -99,25 +98,15 @@ __global__ void k_set_ints(int* __restrict__ p, int64_t n, int v) {
 
 // The frustum's bins, 8 per slab: bin 8 s + j starts at the j-th step of the
 // float recurrence from t_from_step(8 s + near_i).  bins[k] = {start, midpoint}.
-// Counts the slabs whose midpoints do not increase up to the next one's first
-// (steps near the rounding of t) in cnt[CNT_UNORDERED].
-__global__ __launch_bounds__(256) void k_fill_bins(fvc_stepsize_info st, int bz, float2* __restrict__ bins,
-                                                   int* __restrict__ cnt) {
+__global__ __launch_bounds__(256) void k_fill_bins(fvc_stepsize_info st, int bz, float2* __restrict__ bins) {
   const int slab = blockIdx.x * 256 + threadIdx.x;
   if (slab >= bz) return;
-  float t1 = t_from_step(st, (float)(slab * BRICK) + st.near_i), last = -1.0f;
-  bool ordered = true;
+  float t1 = t_from_step(st, (float)(slab * BRICK) + st.near_i);
   for (int j = 0; j < BRICK; j++) {
     const float t0 = t1;
     t1 = t0 + step_dt(st, t0);
-    const float tm = (t0 + t1) * 0.5f;
-    bins[slab * BRICK + j] = make_float2(t0, tm);
-    ordered = ordered && tm > last;
-    last = tm;
+    bins[slab * BRICK + j] = make_float2(t0, (t0 + t1) * 0.5f);
   }
-  const float n0 = t_from_step(st, (float)((slab + 1) * BRICK) + st.near_i);
-  ordered = ordered && (n0 + (n0 + step_dt(st, n0))) * 0.5f > last;
-  if (!ordered) atomicAdd(&cnt[CNT_UNORDERED], 1);
 }
 
 // Tile flags (bytes 0 or 1) are scanned by many blocks, FLAG_RUN flags a
@@ -192,44 +181,18 @@ __global__ __launch_bounds__(256) void k_fill_list(int n_tiles, const uint8_t* _
 // for their slowest; refills with 1 / 4 / 8 / 16 tiles: 1920x1080 19290 / 17780
 // / 17845 / 18530 us, 400x400 of the small scene 13765 / 13885 / 14030 / 14400.
 static const int FILL_TILES = 4;
-// First bin k in [lo, n] whose midpoint exceeds t (n: none), for midpoints
-// that increase: the estimate of the continuous schedule, checked and
-// corrected on the table.
-__device__ __forceinline__ int bin_past(const StepTableView& est, const float2* __restrict__ bins, int lo, int n,
-                                        float t) {
-  const float e = fminf(fmaxf(floorf(step_estimate(est, t) - est.near_i + 0.5f), 0.0f), 1.0e9f);
-  int k = (int)e;
-  k = k < lo ? lo : (k > n ? n : k);
-  while (k > lo && bins[k - 1].y > t) k--;
-  while (k < n && bins[k].y <= t) k++;
-  return k;
-}
-
 // sample_cache_init_first_kernel + sample_cache_init_second_kernel
-// (cache_renderer.cu:83-287): a tile (8 x 8 rays, one wave) goes to the first
-// slab (8 bins) in which a ray has an occupied bin and emits the slab's
-// occupied bins as a compacted stream.
-//
-// Every ray looks for its own first occupied bin once, box by box, and keeps
-// it over the sub-iterations (FillRay::next); the tile's slab is the least of
-// them.  A walk of the whole tile from slab to slab, asking the 64 rays' bins
-// again in each, costs a box query per slab for the slowest ray of every
-// launch: its chain of loads was the kernel's time.  Samples are laid out bin
-// by bin (fill_offsets), so every store of a bin is contiguous over the wave.
-// Measured (all launches of a fill): 1920x1080 of the unbounded scene 5.13 ms
-// walked and reserved by tile, 4.08 searched, 2.5 with FILL_TILES; 400x400 of
-// the small scene 20.6 walked, 6.4 searched.
-//
-// Rays that have ended are asked in every slab the tile visits, and the tile
-// only visits the slabs that no live ray jumps over.  Where an ended ray has
-// an occupied bin before any live one does, the slab depends on those jumps,
-// and the tile walks: after an empty slab it passes the slabs that every live
-// lane's empty box covers (a lane's first bin that is neither in its skip
-// interval nor past its far bound lies at or after step_from_t(min(hi, far))
-// - near_i - 2, two bins of margin for rounding).  It also walks where the
-// midpoints are not ordered.
+// (cache_renderer.cu:83-287): skip empty slabs, emit the occupied samples of
+// the first non-empty one as a compacted stream.  One wave per tile of the
+// alive list (grid-stride).  After an empty slab the wave jumps over the
+// slabs that every live lane's empty box covers: a lane's first bin that is
+// neither in its skip interval nor past its far bound lies at or after
+// step_from_t(min(hi, far)) - near_i - 2 (two bins of margin for rounding).
+// Samples are laid out bin by bin (fill_offsets), so every store of a bin is
+// contiguous over the wave; the wave decides by ballots (a wave sum by
+// shuffles is 6 LDS round trips); LDS holds the scene's cascades only.
 __global__ __launch_bounds__(64 * FILL_TILES) void k_fill_sample(const int* __restrict__ list, const int* __restrict__ cnt,
-                                                    fvc_stepsize_info st, StepTableView est, OccParams occ,
+                                                    fvc_stepsize_info st, OccParams occ,
                                                     ContractParams con, const uint64_t* __restrict__ bf,
                                                     const uint32_t* __restrict__ coarse_g, int bz,
                                                     const float2* __restrict__ bins, V3 o,
@@ -243,8 +206,6 @@ __global__ __launch_bounds__(64 * FILL_TILES) void k_fill_sample(const int* __re
   extern __shared__ uint32_t coarse[];  // nlvl * COARSE_WORDS
   load_coarse(coarse_g, occ.nlvl, coarse);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nb = bz * BRICK;
-  const bool ordered = cnt[CNT_UNORDERED] == 0;
   for (int l0 = blockIdx.x * FILL_TILES; l0 < n_list; l0 += gridDim.x * FILL_TILES) {
     const bool valid = l0 + wave < n_list;  // else the wave repeats a tile and writes nothing
     const int t = list[valid ? l0 + wave : l0];
@@ -257,58 +218,7 @@ __global__ __launch_bounds__(64 * FILL_TILES) void k_fill_sample(const int* __re
     int slab = tile.slab;
     unsigned mask = 0;
     bool any = false;  // some lane has a sample in the slab
-    bool walk = !ordered;
-    if (ordered && slab < bz) {
-      // the ray's first occupied bin (nb: none)
-      int b = sta.next;
-      if (b < slab * BRICK) {
-        b = slab * BRICK;
-        while (b < nb) {
-          const float tm = bins[b].y;
-          if (tm > r.far_) { b = nb; break; }
-          Skip sk = no_skip();
-          if (occ_query(o + tm * d, occ, bf, coarse, rslab, sk)) break;
-          b = in_skip(sk, tm) ? bin_past(est, bins, b + 1, nb, sk.hi) : b + 1;
-        }
-        sta.next = b;
-      }
-      const int s_live = wave_min(alive ? b : nb) / BRICK, s_ended = wave_min(alive ? nb : b) / BRICK;
-      if (s_ended < s_live) {
-        walk = true;
-      } else if (s_live < bz) {
-        any = true;
-        slab = s_live;
-        if (b / BRICK == slab) {
-          // the ray's other bins of the slab, their words loaded together
-          OccCell cell[BRICK];
-          uint32_t at[BRICK];
-          uint64_t word[BRICK];
-          const int first = b % BRICK;
-#pragma unroll
-          for (int j = 1; j < BRICK; j++) {
-            cell[j] = occ_cell(o + bins[slab * BRICK + j].y * d, occ, coarse);
-            at[j] = occ_index(cell[j]);
-            word[j] = bf[cell[j].block ? at[j] >> 6 : 0u];
-          }
-          mask = 1u << first;
-#pragma unroll
-          for (int j = 1; j < BRICK; j++)
-            if (j > first && !(bins[slab * BRICK + j].y > r.far_) && cell[j].block &&
-                ((word[j] >> (at[j] & 63u)) & 1u))
-              mask |= 1u << j;
-        }
-        if (bins[slab * BRICK + BRICK - 1].y > r.far_) alive = false;
-      } else {
-        // no sample is left: the tile ends after the slab in which its last live ray passes far
-        const int past = alive ? bin_past(est, bins, slab * BRICK, nb, r.far_) / BRICK + 1 : 0;
-        const int end = -wave_min(-past);
-        slab = end < bz ? end : bz;
-        alive = false;
-      }
-    } else if (slab >= bz) {  // beyond the frustum: the column ends
-      alive = false;
-    }
-    if (walk) {
+    {
       Skip sk = no_skip();
       while (__ballot(alive) != 0) {
         if (slab >= bz) {
@@ -722,7 +632,6 @@ void cache_fill(Renderer& r, const fvc_raymarch_info& rm, fvc_init_stats* stats,
   r.f_tiles.ensure((int64_t)n_tiles * sizeof(FillTile));
   r.f_list.ensure((int64_t)n_tiles * sizeof(int));
   r.f_bins.ensure((int64_t)C.bz * BRICK * sizeof(float2));
-  const StepTableView est = step_view(rm.stepsize_info);
   const unsigned n_flag_blocks = (unsigned)((n_tiles + FLAG_BLOCK - 1) / FLAG_BLOCK);
   r.f_alive8.ensure((int64_t)n_flag_blocks * FLAG_BLOCK);
   r.f_alloc8.ensure((int64_t)n_flag_blocks * FLAG_BLOCK);
@@ -745,7 +654,7 @@ void cache_fill(Renderer& r, const fvc_raymarch_info& rm, fvc_init_stats* stats,
                        n_table, -1);
     hipLaunchKernelGGL(k_set_ints, dim3(1), dim3(FILL_LOG), 0, s, cnt, (int64_t)FILL_LOG, 0);
     hipLaunchKernelGGL(k_fill_bins, dim3((C.bz + 255) / 256), dim3(256), 0, s, rm.stepsize_info, C.bz,
-                       r.f_bins.as<float2>(), cnt);
+                       r.f_bins.as<float2>());
     hipLaunchKernelGGL(k_fill_init, dim3(n_tiles), dim3(64), 0, s, rm, cvt(m.scene.aabb_from),
                        cvt(m.scene.aabb_to), C.bx, r.f_rays.as<FillRay>(), r.f_ray_t.as<float>(), r.f_state.as<FillState>(),
                        r.f_tiles.as<FillTile>(), r.f_alive8.as<uint8_t>());
@@ -762,7 +671,7 @@ void cache_fill(Renderer& r, const fvc_raymarch_info& rm, fvc_init_stats* stats,
     h.list = P.end(ev, s, "fill_list");
     ev = P.begin(s);
     hipLaunchKernelGGL(k_fill_sample, dim3((unsigned)std::min((n_tiles + FILL_TILES - 1) / FILL_TILES, 65536)), dim3(64 * FILL_TILES), (size_t)m.occ.nlvl * COARSE_WORDS * sizeof(uint32_t), s,
-                       r.f_list.as<int>(), cnt, rm.stepsize_info, est, m.occ, m.con, m.bitfield.as<uint64_t>(),
+                       r.f_list.as<int>(), cnt, rm.stepsize_info, m.occ, m.con, m.bitfield.as<uint64_t>(),
                        m.coarse.as<uint32_t>(), C.bz, r.f_bins.as<float2>(), translation(rm.cam_info.cam2world),
                        r.f_rays.as<FillRay>(), r.f_state.as<FillState>(), r.f_tiles.as<FillTile>(), r.f_pos.as<float>(),
                        cnt + CNT_SAMPLES, split ? r.f_dir.as<float>() : nullptr, r.f_alive8.as<uint8_t>());

@@ -65,7 +65,7 @@ static const int COMPOSITE_BATCH = 16;
 
 // slots of Renderer::counters
 enum { CNT_ALIVE = 0, CNT_SAMPLES = 1, CNT_CACHE = 2, CNT_STEPS = 3, CNT_TILES = 4, CNT_OVERFLOW = 6,
-       CNT_UNORDERED = 7, CNT_SLOTS = 8 /* and 9 */ };
+       CNT_SLOTS = 8 /* and 9 */ };
 
 // Device control block of a frame's sub-iteration loop (also in
 // Renderer::counters): one record per iteration, all zero when the frame

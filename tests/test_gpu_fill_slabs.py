@@ -1,8 +1,7 @@
-"""The fill's search for a tile's next slab: where rays ended before their
-neighbours (opaque ones still have samples in the tile's slabs, past ones have
-none), on ragged tile edges, and where steps near the rounding of t leave bin
-midpoints unordered (the tile is then walked slab by slab).  Index work is the
-oracle's bit for bit."""
+"""The fill's slabs and sample order: where rays ended before their neighbours
+(opaque ones still have samples in the tile's slabs, past ones have none), on
+ragged tile edges, and where steps near the rounding of t leave bin midpoints
+unordered.  Index work is the oracle's bit for bit."""
 import numpy as np
 import pytest
 
