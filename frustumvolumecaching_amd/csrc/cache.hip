@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void k_fill_bins(fvc_stepsize_info st, int bz,
 // thread: a block counts the flags before its own by itself (all of them lie
 // in L2), so the scan is one launch without a chain between blocks.  One block
 // for all tiles cost 16 us a launch at 1920x1080 (32400 tiles), mostly its
-// scattered stores by one CU; now 4.
+// scattered stores by one CU; now 5.
 static const int FLAG_RUN = 8, FLAG_BLOCK = 256 * FLAG_RUN;  // flags per thread and block
 __device__ __forceinline__ int block_excl_sum(int v, int& total) {
   __shared__ int s_w[4];
@@ -176,10 +176,11 @@ __global__ __launch_bounds__(256) void k_fill_list(int n_tiles, const uint8_t* _
 
 // Tiles per block of k_fill_sample.  A returning atomic on one address takes
 // 11.5 ns, whoever asks (95.7 us for 8100 blocks, 371 for 32400, one to three
-// counters alike), so a reservation per tile was the kernel's time: 12000
-// tiles with samples in a launch at 1920x1080, 135 us.  More tiles wait longer
-// for their slowest; refills with 1 / 4 / 8 / 16 tiles: 1920x1080 19290 / 17780
-// / 17845 / 18530 us, 400x400 of the small scene 13765 / 13885 / 14030 / 14400.
+// counters alike), so a reservation per tile is at least 135 us a launch at
+// 1920x1080 (12000 tiles with samples).  More tiles wait longer for their
+// slowest; refills with 1 / 4 / 8 / 16 tiles, measured with a shorter search
+// for the slab: 1920x1080 19290 / 17780 / 17845 / 18530 us, 400x400 of the small
+// scene 13765 / 13885 / 14030 / 14400.
 static const int FILL_TILES = 4;
 // sample_cache_init_first_kernel + sample_cache_init_second_kernel
 // (cache_renderer.cu:83-287): skip empty slabs, emit the occupied samples of
@@ -190,7 +191,10 @@ static const int FILL_TILES = 4;
 // step_from_t(min(hi, far)) - near_i - 2 (two bins of margin for rounding).
 // Samples are laid out bin by bin (fill_offsets), so every store of a bin is
 // contiguous over the wave; the wave decides by ballots (a wave sum by
-// shuffles is 6 LDS round trips); LDS holds the scene's cascades only.
+// shuffles is 6 LDS round trips); LDS holds the scene's cascades only.  Bound
+// by the slowest tile's chain of box queries.  Measured per launch: 1920x1080
+// of the unbounded scene 179 -> 127 us; 400x400 of the small scene 195 -> 170
+// by the ballots, 209 with four tiles a block (its refill 31.4 -> 29.0 ms).
 __global__ __launch_bounds__(64 * FILL_TILES) void k_fill_sample(const int* __restrict__ list, const int* __restrict__ cnt,
                                                     fvc_stepsize_info st, OccParams occ,
                                                     ContractParams con, const uint64_t* __restrict__ bf,
